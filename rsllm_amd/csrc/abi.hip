@@ -491,6 +491,22 @@ int lora_down_compute(float *out, size_t out_len, const uint8_t *w, size_t strid
         return ok();
     }
     hipError_t e = hipErrorNotSupported;
+    // Prompts: the many-token GEMM, once the 16-token passes below would make
+    // more than about five workgroups per two CUs, or from 256 tokens (which
+    // pay for its longer workgroups on few rows): passes against GEMM, 8 x
+    // [1024 x 4096] Q8_0 52 vs 54 us at 64 tokens, 74 vs 56 at 96, 236 vs 83
+    // at 300; 4 x [512 x 2048] 23 vs 32 at 96, 47 vs 35 at 300; 16 x [256 x
+    // 1024] 20 vs 23 at 96, 27 vs 25 at 160; 8 x [128 x 4096] 44 vs 54 at
+    // 160, 78 vs 59 at 300.
+    const long passes_wg = ((long)T + 15) / 16 * ((long)G * R / 64);
+    if (!group_layout && (passes_wg >= 640 || T >= 256) && T > 32 &&
+        gemm_exact_supported(dtype, T, D, G, R)) {
+        HIP_TRY(sc.xq.ensure(gemm_exact_scratch_bytes(T, D, G)), "hipMalloc");
+        e = launch_gemm_exact(dtype, w, stride * n_groups, x, (uint8_t *)sc.xq.p, out, T, D, G, R,
+                              tout, s);
+        if (e == hipSuccess) return ok();
+        if (e != hipErrorNotSupported) return dev_err(e, "gemm_exact");
+    }
     // 9 or more tokens of the matrix-core formats: one pass over the stacked
     // matrix per 16 tokens, on the matrix cores
     if (!group_layout && lora_mfma_supported(dtype, T, D, G, R)) {

@@ -185,6 +185,18 @@ hipError_t launch_lora_mfma(uint32_t dtype, const uint8_t *w, size_t w_bytes, co
                             int x_stride, float *y, int y_stride, uint8_t *scratch, int n_tok,
                             int D, int G, int R, hipStream_t s);
 
+// gemm_exact.hip: y[t * y_stride + g * group_rows + r] = sum_i W[g *
+// group_rows + r, i] x[(t * groups + g) * in_dim + i] for a matrix of groups *
+// group_rows rows (device layout as one matrix), the weights exact and the
+// activations as hi + lo f16. `scratch` holds gemm_exact_scratch_bytes bytes.
+// Q8_0; hipErrorNotSupported outside gemm_exact_supported or where w or x is
+// not 16-byte aligned.
+bool gemm_exact_supported(uint32_t dtype, int n_tok, int in_dim, int groups, int group_rows);
+size_t gemm_exact_scratch_bytes(int n_tok, int in_dim, int groups);
+hipError_t launch_gemm_exact(uint32_t dtype, const uint8_t *w, size_t w_bytes, const float *x,
+                             uint8_t *scratch, float *y, int n_tok, int in_dim, int groups,
+                             int group_rows, int y_stride, hipStream_t s);
+
 // prefill.hip: out[t, o] = sum_i deq(W)[o, i] * x[t, i] for a raw GGUF Q4_K
 // weight W [out_dim x in_dim] and bf16 activations x [n_tok x in_dim]
 // (n_tok x out_dim fp32 output, overwritten). `scratch` holds

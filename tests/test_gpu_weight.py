@@ -257,3 +257,25 @@ def test_grouped_lora_down_matrix_cores(oracle, hip, dtype, n_groups, group_dim,
     err = rel_err(got.reshape(n_tok, -1)[toks], want)
     print(f"lora_down mfma {G(dtype).name} T={n_tok} {n_groups}x[{rank}x{group_dim}]: rel err {err:.3e}")
     assert err <= REL_TOL
+
+
+@pytest.mark.parametrize("n_groups,group_dim,rank,n_tok", [
+    (1, 256, 1, 256),       # one row, one tile of K
+    (3, 512, 384, 257),     # ranks of one and a half row blocks, a ragged token tile
+    (2, 768, 257, 300),     # one row into the second block, K of three tiles
+    (8, 1024, 512, 161),    # many row blocks below 256 tokens
+    (5, 256, 128, 1000),    # several token tiles per group
+])
+def test_grouped_lora_down_many_token_gemm(oracle, hip, n_groups, group_dim, rank, n_tok):
+    """Q8_0 prompts on the many-token GEMM: exact weights, activations to
+    about 2^-22, fp32 sums of group_dim terms in a few hundred additions, so
+    2e-5 of the largest output covers any order of summation."""
+    w, x = grouped_case(G.Q8_0, n_tok, n_groups, group_dim, rank, 900 + n_tok)
+    x[n_tok // 2] *= 1e4  # a token of another scale
+    toks = np.unique(np.array([0, 15, 16, 47, 48, n_tok // 2, n_tok - 1]))
+    want = oracle_grouped(oracle, w, x, toks, n_groups, group_dim, rank, G.Q8_0)
+    got = np.full(n_tok * n_groups * rank, np.nan, np.float32)
+    hip.matmul_grouped_lora_down(got, w, x.reshape(-1), n_tok, n_groups, group_dim, rank, G.Q8_0)
+    assert not np.isnan(got).any()
+    for k, t in enumerate(toks):
+        assert rel_err(got.reshape(n_tok, -1)[t], want[k]) <= 2e-5
