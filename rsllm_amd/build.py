@@ -24,8 +24,8 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "librsllm_hip.so")
 
-SOURCES = ["abi.hip", "dequant.hip", "gemv.hip", "gemv_mfma.hip", "gemm_exact.hip", "prefill.hip",
-           "moe.hip", "q8_int8.hip", "residency.hip", "probe.hip"]
+SOURCES = ["abi.hip", "dequant.hip", "gemv.hip", "gemv_mfma.hip", "gemm_exact.hip", "moe_gemm.hip",
+           "prefill.hip", "moe.hip", "q8_int8.hip", "residency.hip", "probe.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -49,6 +49,7 @@ EXTRA_FLAGS = {
     "prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "gemv_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "gemm_exact.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "moe_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

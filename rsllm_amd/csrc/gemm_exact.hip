@@ -32,42 +32,10 @@
 // a ring of four 64-element steps, 89 us: a row's 64 bytes and its scales per
 // step touch three times the lines of a whole tile. 8 wavefronts of four row
 // tiles, 77 us.)
+#include "buffer_lds.h"
 #include "mfma_formats.h"
 
 namespace rsllm_hip {
-
-// A raw-buffer resource in scalar registers (base, size in bytes).
-typedef uint32_t xg_rsrc __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ xg_rsrc xg_make_rsrc(const void *p, uint32_t bytes) {
-    const uint64_t a = (uint64_t)(size_t)p;
-    return xg_rsrc{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
-                   (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32) & 0xFFFF),
-                   (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
-}
-// LDS byte address of a pointer into the workgroup's LDS.
-__device__ __forceinline__ uint32_t xg_lds(const void *p) {
-    return (uint32_t)(size_t)(const __attribute__((address_space(3))) void *)p;
-}
-// 16 bytes per lane from the buffer to LDS: lane i's bytes at voff + soff go to lds
-// + 16 i (lds uniform); a lane whose bytes lie past the resource moves zeros
-// without an access. Written by hand, so the compiler adds no wait for it
-// before LDS reads (with the builtin it waits for every copy in flight):
-// xg_barrier orders each copy against its readers. M0 is restored; the
-// memory clobber keeps LDS accesses on their side.
-__device__ __forceinline__ void xg_dma16(const xg_rsrc &r, uint32_t voff, uint32_t soff, uint32_t lds) {
-    const uint32_t ls = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds);
-    uint32_t saved;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
-                 "buffer_load_dwordx4 %1, %2, %4 offen lds\n\ts_mov_b32 m0, %0"
-                 : "=&s"(saved)
-                 : "v"(voff), "s"(r), "s"(ls), "s"(soff)
-                 : "memory");
-}
-// All but this wavefront's N newest copies have landed and its LDS accesses
-// are done, then everyone's.
-template <int N> __device__ __forceinline__ void xg_barrier() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
 
 // Per format: a row's tile of 256 elements is PR 16-byte pieces (PR odd, so
 // 16 rows at a stride of PR pieces start on distinct LDS bank groups). The
@@ -160,8 +128,8 @@ __global__ __launch_bounds__(64 * kXgWaves) void k_xg(const uint8_t *__restrict_
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wv & (kXgWR - 1), kg = wv / kXgWR;
     const int nt256 = sh.in_dim / 256, ns = 4 * nt256;  // tiles, steps
-    const xg_rsrc rw = xg_make_rsrc(w, sh.w_bytes), rx = xg_make_rsrc(xh, sh.x_bytes);
-    const uint32_t lds0 = xg_lds(smem);
+    const bl_rsrc rw = bl_make_rsrc(w, sh.w_bytes), rx = bl_make_rsrc(xh, sh.x_bytes);
+    const uint32_t lds0 = bl_lds(smem);
     const uint8_t *const wbuf = smem + kXgRing * G::X;  // after the activations' ring
 
     // Copies, the same number from every wavefront (those past the last
@@ -186,18 +154,18 @@ __global__ __launch_bounds__(64 * kXgWaves) void k_xg(const uint8_t *__restrict_
                 16u * (uint32_t)((lane & 15) ^ (tr & 15));
     }
     auto dma_w = [&](int t) {
-        const xg_rsrc r = {rw[0], rw[1], t < nt256 ? rw[2] : 0u, rw[3]};
+        const bl_rsrc r = {rw[0], rw[1], t < nt256 ? rw[2] : 0u, rw[3]};
 #pragma unroll
         for (int p = 0; p < G::WI; p++)
-            xg_dma16(r, wo[p], (uint32_t)t * (16u * G::PR),
+            bl_dma16(r, wo[p], (uint32_t)t * (16u * G::PR),
                      lds0 + (uint32_t)(kXgRing * G::X) + 1024u * (uint32_t)min(wv + kXgWaves * p, G::WN - 1));
     };
     auto dma_x = [&](int s) {
         const uint32_t dst = lds0 + (uint32_t)((s & (kXgRing - 1)) * G::X);
-        const xg_rsrc r = {rx[0], rx[1], s < ns ? rx[2] : 0u, rx[3]};
+        const bl_rsrc r = {rx[0], rx[1], s < ns ? rx[2] : 0u, rx[3]};
 #pragma unroll
         for (int p = 0; p < G::XI; p++)
-            xg_dma16(r, xo[p], 256u * (uint32_t)s,
+            bl_dma16(r, xo[p], 256u * (uint32_t)s,
                      dst + 1024u * (uint32_t)min(wv + kXgWaves * p, G::XN - 1));
     };
     f32x4 acc[RT][NT];
@@ -266,7 +234,7 @@ __global__ __launch_bounds__(64 * kXgWaves) void k_xg(const uint8_t *__restrict_
             // the tile's last step the next tile's weights; newer copies may
             // still be in flight. (Order of issue: steps' activations, a
             // tile's weights after those issued in its first step.)
-            xg_barrier<(u == 1 || u == 2) ? G::XI + G::WI : G::XI>();
+            bl_barrier<(u == 1 || u == 2) ? G::XI + G::WI : G::XI>();
             dma_x(s + 3);
             if constexpr (u == 0) dma_w((s >> 2) + 1);
             if constexpr (KG == 0) {
@@ -311,10 +279,10 @@ __global__ __launch_bounds__(64 * kXgWaves) void k_xg(const uint8_t *__restrict_
     dma_x(0);
     dma_x(1);
     dma_x(2);
-    xg_barrier<2 * G::XI>();
+    bl_barrier<2 * G::XI>();
     if (kg == 0) run(std::integral_constant<int, 0>{});
     else run(std::integral_constant<int, 1>{});
-    xg_barrier<0>();
+    bl_barrier<0>();
     // the K groups' sums: group 0 keeps the lower half of each wavefront's
     // (row tile, column tile) pairs, group 1 the upper
     constexpr int PAIRS = RT * NT, H0 = G::H0;

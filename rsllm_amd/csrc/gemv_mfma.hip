@@ -809,10 +809,13 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_mfo(const uint8_t *__restrict_
 // one workgroup of TH threads, the row read once when it fits in
 // registers): val4(i) gives elements i .. i + 3 of the column's row; the
 // column's pieces go to both planes of the image at xb (the lo plane
-// `plane` halves after the hi plane; 0: in_dim * ntp), 2^-e to *us.
+// `plane` halves after the hi plane; 0: in_dim * ntp), 2^-e to *us, and with
+// `sums` (in_dim a multiple of 256) the column's sub-block sums there
+// (moe_gemm_sums).
 template <class F, int TH = kMfxThreads, class V>
 __device__ __forceinline__ void mf_x_column(V val4, int in_dim, int t, _Float16 *__restrict__ xb,
-                                            float *__restrict__ us, int ntp, size_t plane = 0) {
+                                            float *__restrict__ us, int ntp, size_t plane = 0,
+                                            _Float16 *__restrict__ sums = nullptr) {
     __shared__ float red[TH / 64];
     const int tid = threadIdx.x;
     const int n8 = in_dim / 8;
@@ -823,6 +826,21 @@ __device__ __forceinline__ void mf_x_column(V val4, int in_dim, int t, _Float16 
         const size_t slot = ((size_t)(s * 4 + j) * 4 + q) * ntp + t;
         *reinterpret_cast<uint4 *>(xb + slot * 8) = hi;
         *reinterpret_cast<uint4 *>(xb + plane + slot * 8) = lo;
+    };
+    auto emit = [&](int i, const float4 &a, const float4 &b, float up) {
+        uint4 hi, lo;
+        hilo8(a, b, up, hi, lo);
+        store(i, hi, lo);
+        if (sums) {  // two neighbouring threads hold a sub-block of 16
+            float s = ((a.x + a.y) + (a.z + a.w)) + ((b.x + b.y) + (b.z + b.w));
+            s = (s + __shfl_xor(s, 1, 64)) * (up * 0.0625f);
+            if ((i & 1) == 0) {
+                const _Float16 h = (_Float16)s;
+                _Float16 *p = sums + (i >> 5) * 32 + ((i >> 1) & 15);
+                p[0] = h;
+                p[16] = (_Float16)(s - (float)h);
+            }
+        }
     };
     // pieces read once (kept in registers) when the row fits
     const bool cached = n8 <= TH * kMfxCache;
@@ -848,18 +866,10 @@ __device__ __forceinline__ void mf_x_column(V val4, int in_dim, int t, _Float16 
 #pragma unroll
         for (int r = 0; r < kMfxCache; r++) {
             const int i = tid + r * TH;
-            if (i < n8) {
-                uint4 hi, lo;
-                hilo8(c[r][0], c[r][1], up, hi, lo);
-                store(i, hi, lo);
-            }
+            if (i < n8) emit(i, c[r][0], c[r][1], up);
         }
     } else {
-        for (int i = tid; i < n8; i += TH) {
-            uint4 hi, lo;
-            hilo8(val4(8 * i), val4(8 * i + 4), up, hi, lo);
-            store(i, hi, lo);
-        }
+        for (int i = tid; i < n8; i += TH) emit(i, val4(8 * i), val4(8 * i + 4), up);
     }
 }
 
@@ -869,7 +879,8 @@ __device__ __forceinline__ void mf_x_column(V val4, int in_dim, int t, _Float16 
 template <class F, bool SWIGLU, int TH>
 __device__ __forceinline__ void mfg_row(const float *__restrict__ x, const float *__restrict__ hu,
                                         int r, float clamp, _Float16 *__restrict__ xh,
-                                        float *__restrict__ unscale, int in_dim) {
+                                        float *__restrict__ unscale, int in_dim,
+                                        _Float16 *__restrict__ sums) {
     const float *xt = x + (size_t)r * in_dim;
     const float *ut = hu + (SWIGLU ? (size_t)r * in_dim : 0);
     auto val4 = [&](int i) {
@@ -883,7 +894,8 @@ __device__ __forceinline__ void mfg_row(const float *__restrict__ x, const float
     };
     // hi of piece p at halves 16 p, lo 8 halves later: two "columns" per
     // piece with the lo plane 8 halves after the hi one
-    mf_x_column<F, TH>(val4, in_dim, 0, xh + (size_t)r * 2 * in_dim, unscale + r, 2, 8);
+    mf_x_column<F, TH>(val4, in_dim, 0, xh + (size_t)r * 2 * in_dim, unscale + r, 2, 8,
+                       sums ? sums + (size_t)r * (in_dim >> 3) : nullptr);
 }
 
 // The SwiGLU image of the down projection: one workgroup per slot.
@@ -892,10 +904,11 @@ __global__ __launch_bounds__(TH) void k_mfg_xs(const float *__restrict__ hg,
                                                const float *__restrict__ hu,
                                                const int *__restrict__ n_rows, float clamp,
                                                _Float16 *__restrict__ xh,
-                                               float *__restrict__ unscale, int in_dim) {
+                                               float *__restrict__ unscale, int in_dim,
+                                               _Float16 *__restrict__ sums) {
     const int r = blockIdx.x;
     if (r >= *n_rows) return;
-    mfg_row<F, true, TH>(hg, hu, r, clamp, xh, unscale, in_dim);
+    mfg_row<F, true, TH>(hg, hu, r, clamp, xh, unscale, in_dim, sums);
 }
 
 // The first launch of the route: workgroup 0 runs the routing (when `route`;
@@ -908,7 +921,8 @@ __global__ __launch_bounds__(kScanThreads) void k_mfg_route_x(MoeRoute1Args ra, 
                                                               const float *__restrict__ x,
                                                               _Float16 *__restrict__ xh,
                                                               float *__restrict__ unscale,
-                                                              int in_dim) {
+                                                              int in_dim,
+                                                              _Float16 *__restrict__ sums) {
     extern __shared__ int sh[];  // routing: 2 n_expert ints
     __shared__ int ep[kRoute1Pairs];
     __shared__ int part[kScanThreads];
@@ -918,7 +932,7 @@ __global__ __launch_bounds__(kScanThreads) void k_mfg_route_x(MoeRoute1Args ra, 
         return;
     }
     mfg_row<F, false, kScanThreads>(x, nullptr, (int)blockIdx.x - (route ? 1 : 0), 0.f, xh, unscale,
-                                    in_dim);
+                                    in_dim, sums);
 }
 
 // ---- grouped LoRA-down on the matrix cores ----------------------------------------
@@ -1511,9 +1525,11 @@ size_t moe_mfma_scratch_bytes(int n_pairs, int n_expert, int n_embd, int n_ff) {
     const int bw = mfg_width(n_pairs, n_expert);
     auto al = [](size_t n) { return (n + 255) / 256 * 256; };
     // the batch list, then the x image (at most n_pairs tokens) and the
-    // SwiGLU image (one row per slot), two f16 planes and a scale per row
+    // SwiGLU image (one row per slot), two f16 planes, sub-block sums and a
+    // scale per row
     return mfg_batch_bytes(n_pairs, n_expert, bw) + al((size_t)n_pairs * n_embd * 4) +
-           al((size_t)n_pairs * 4) + al((size_t)n_pairs * n_ff * 4) + al((size_t)n_pairs * 4);
+           al((size_t)n_pairs * n_embd / 4) + al((size_t)n_pairs * 4) +
+           al((size_t)n_pairs * n_ff * 4) + al((size_t)n_pairs * n_ff / 4) + al((size_t)n_pairs * 4);
 }
 
 bool moe_mfma_fits(int n_pairs, int n_embd, int n_ff) {
@@ -1525,10 +1541,21 @@ bool moe_mfma_fits(int n_pairs, int n_embd, int n_ff) {
 // the batches, against the per-row image xh of n_rows rows.
 template <class F>
 static hipError_t mfg_gemv(const uint8_t *w0, const uint8_t *w1, size_t w_stride,
-                           const _Float16 *xh, const float *us, int n_rows, const int *tok,
-                           const MfgBatch *bat, const int *n_bat, int max_b, float *y0, float *y1,
-                           int in_dim, int out_dim, int bw, hipStream_t s) {
+                           const _Float16 *xh, const _Float16 *sums, const float *us, int n_rows,
+                           const int *tok, const MfgBatch *bat, const int *n_bat, int max_b,
+                           float *y0, float *y1, int in_dim, int out_dim, int bw, hipStream_t s) {
     const uint32_t plane = (uint32_t)((size_t)n_rows * in_dim * 2);
+    // the DS-V4 expert formats, 16-slot batches: weights and activations
+    // staged through LDS
+    if constexpr (std::is_same<F, MIQ2>::value || std::is_same<F, MQ2K>::value) {
+        if (bw == kMfgBatch) {
+            const uint32_t dt = std::is_same<F, MIQ2>::value ? T_IQ2_XXS : T_Q2_K;
+            const hipError_t e = launch_moe_gemm16(dt, w0, w1, w_stride, xh, (size_t)n_rows * in_dim * 4,
+                                                   sums, sums ? (size_t)n_rows * (in_dim / 4) : 0, us,
+                                                   tok, bat, n_bat, max_b, y0, y1, in_dim, out_dim, s);
+            if (e != hipErrorNotSupported) return e;
+        }
+    }
     // weights staged through LDS where the layout allows (16-byte aligned
     // expert matrices, in_dim a multiple of 1024, of 2048 for Q6_K)
     // (Q2_K and IQ2_XXS: 8-slot batches only; with 16-slot batches the
@@ -1576,16 +1603,16 @@ static hipError_t mfg_gemv(const uint8_t *w0, const uint8_t *w1, size_t w_stride
 template <class F>
 static hipError_t mfg_swiglu_image(const float *hg, const float *hu, const int *n_rows,
                                    int n_alloc, float clamp, _Float16 *xh, float *us, int in_dim,
-                                   hipStream_t s) {
+                                   _Float16 *sums, hipStream_t s) {
     // 256 threads for rows of up to 2048 elements (one 8-element piece per
     // thread), 512 up to 8192, else kMfxThreads
     const dim3 g((unsigned)n_alloc);
     if (in_dim <= 2048)
-        k_mfg_xs<F, 256><<<g, 256, 0, s>>>(hg, hu, n_rows, clamp, xh, us, in_dim);
+        k_mfg_xs<F, 256><<<g, 256, 0, s>>>(hg, hu, n_rows, clamp, xh, us, in_dim, sums);
     else if (in_dim <= 8192)
-        k_mfg_xs<F, 512><<<g, 512, 0, s>>>(hg, hu, n_rows, clamp, xh, us, in_dim);
+        k_mfg_xs<F, 512><<<g, 512, 0, s>>>(hg, hu, n_rows, clamp, xh, us, in_dim, sums);
     else
-        k_mfg_xs<F, kMfxThreads><<<g, kMfxThreads, 0, s>>>(hg, hu, n_rows, clamp, xh, us, in_dim);
+        k_mfg_xs<F, kMfxThreads><<<g, kMfxThreads, 0, s>>>(hg, hu, n_rows, clamp, xh, us, in_dim, sums);
     return hipGetLastError();
 }
 
@@ -1600,27 +1627,29 @@ static hipError_t mfg_swiglu_image(const float *hg, const float *hu, const int *
     }
 
 static hipError_t mfg_gemv_dt(uint32_t dt, const uint8_t *w0, const uint8_t *w1, size_t w_stride,
-                              const _Float16 *xh, const float *us, int n_rows, const int *tok,
-                              const MfgBatch *bat, const int *n_bat, int max_b, float *y0,
-                              float *y1, int in_dim, int out_dim, int bw, hipStream_t s) {
-    MFG_DT(dt, mfg_gemv<F>(w0, w1, w_stride, xh, us, n_rows, tok, bat, n_bat, max_b, y0, y1,
+                              const _Float16 *xh, const _Float16 *sums, const float *us,
+                              int n_rows, const int *tok, const MfgBatch *bat, const int *n_bat,
+                              int max_b, float *y0, float *y1, int in_dim, int out_dim, int bw,
+                              hipStream_t s) {
+    MFG_DT(dt, mfg_gemv<F>(w0, w1, w_stride, xh, sums, us, n_rows, tok, bat, n_bat, max_b, y0, y1,
                            in_dim, out_dim, bw, s))
 }
 
 static hipError_t mfg_swiglu_image_dt(uint32_t dt, const float *hg, const float *hu,
                                       const int *n_rows, int n_alloc, float clamp, _Float16 *xh,
-                                      float *us, int in_dim, hipStream_t s) {
-    MFG_DT(dt, mfg_swiglu_image<F>(hg, hu, n_rows, n_alloc, clamp, xh, us, in_dim, s))
+                                      float *us, int in_dim, _Float16 *sums, hipStream_t s) {
+    MFG_DT(dt, mfg_swiglu_image<F>(hg, hu, n_rows, n_alloc, clamp, xh, us, in_dim, sums, s))
 }
 
 static hipError_t mfg_route_x_dt(uint32_t dt, const MoeRoute1Args *ra, MfgBatch *bat, int *n_bat,
                                  int bw, const float *x, int n_tok, _Float16 *xh, float *us,
-                                 int in_dim, hipStream_t s) {
+                                 int in_dim, _Float16 *sums, hipStream_t s) {
     const MoeRoute1Args none{};
     const unsigned grid = (unsigned)n_tok + (ra ? 1u : 0u);
     const size_t lds = ra ? (size_t)ra->n_expert * 8 : 0;
     MFG_DT(dt, (k_mfg_route_x<F><<<grid, kScanThreads, lds, s>>>(ra ? *ra : none, bat, n_bat, bw,
-                                                                 ra ? 1 : 0, x, xh, us, in_dim),
+                                                                 ra ? 1 : 0, x, xh, us, in_dim,
+                                                                 sums),
                 hipGetLastError()))
 }
 #undef MFG_DT
@@ -1646,22 +1675,26 @@ hipError_t launch_moe_mfma(uint32_t dt_gu, uint32_t dt_d, const uint8_t *gate, c
         return r;
     };
     _Float16 *xh1 = reinterpret_cast<_Float16 *>(take((size_t)n_pairs * n_embd * 4));
+    _Float16 *sm1 = reinterpret_cast<_Float16 *>(take((size_t)n_pairs * n_embd / 4));
     float *us1 = reinterpret_cast<float *>(take((size_t)n_pairs * 4));
     _Float16 *xh2 = reinterpret_cast<_Float16 *>(take((size_t)n_pairs * n_ff * 4));
+    _Float16 *sm2 = reinterpret_cast<_Float16 *>(take((size_t)n_pairs * n_ff / 4));
     float *us2 = reinterpret_cast<float *>(take((size_t)n_pairs * 4));
+    if (bw != kMfgBatch || !moe_gemm_sums(dt_gu)) sm1 = nullptr;
+    if (bw != kMfgBatch || !moe_gemm_sums(dt_d)) sm2 = nullptr;
     hipError_t e;
     // routing (when given) and the x image in one launch
-    if ((e = mfg_route_x_dt(dt_gu, route, bat, n_bat, bw, x, n_tok, xh1, us1, n_embd, s)) !=
+    if ((e = mfg_route_x_dt(dt_gu, route, bat, n_bat, bw, x, n_tok, xh1, us1, n_embd, sm1, s)) !=
         hipSuccess)
         return e;
-    if ((e = mfg_gemv_dt(dt_gu, gate, up, gu_stride, xh1, us1, n_tok, slot_tok, bat, n_bat, max_b,
+    if ((e = mfg_gemv_dt(dt_gu, gate, up, gu_stride, xh1, sm1, us1, n_tok, slot_tok, bat, n_bat, max_b,
                          hg, hu, n_embd, n_ff, bw, s)) != hipSuccess)
         return e;
     // off[n_expert]: the routed slot count
     if ((e = mfg_swiglu_image_dt(dt_d, hg, hu, off + n_expert, n_pairs, clamp, xh2, us2, n_ff,
-                                 s)) != hipSuccess)
+                                 sm2, s)) != hipSuccess)
         return e;
-    return mfg_gemv_dt(dt_d, down, nullptr, d_stride, xh2, us2, n_pairs, nullptr, bat, n_bat,
+    return mfg_gemv_dt(dt_d, down, nullptr, d_stride, xh2, sm2, us2, n_pairs, nullptr, bat, n_bat,
                        max_b, yd, nullptr, n_ff, n_embd, bw, s);
 }
 

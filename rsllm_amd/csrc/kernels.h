@@ -172,6 +172,20 @@ hipError_t launch_moe_mfma(uint32_t dt_gu, uint32_t dt_d, const uint8_t *gate, c
                            int n_expert, float *hg, float *hu, float *yd, uint8_t *scratch,
                            int n_embd, int n_ff, float clamp, hipStream_t s);
 
+// moe_gemm.hip: the grouped GEMV of one matrix pair (w1 given) or matrix over
+// 16-slot batches against the per-row image xh (x_bytes bytes; row r at byte
+// 4 r in_dim, scaled back by us[r]; column c of a batch reads row tok[first +
+// c], or first + c without tok), weights and activations staged through LDS.
+// moe_gemm_sums(dtype): the image needs sub-block sums beside it, at `sums`
+// (s_bytes bytes): row r's in_dim / 256 blocks of 32 f16 values, 2^-4 of the
+// scaled row's sums over 16 elements as 16 hi then 16 lo planes.
+// hipErrorNotSupported for formats, alignments or in_dim it does not take.
+inline bool moe_gemm_sums(uint32_t dtype) { return dtype == T_Q2_K; }
+hipError_t launch_moe_gemm16(uint32_t dtype, const uint8_t *w0, const uint8_t *w1, size_t w_stride,
+                             const void *xh, size_t x_bytes, const void *sums, size_t s_bytes,
+                             const float *us, const int *tok, const MfgBatch *bat, const int *n_bat, int max_b, float *y0, float *y1,
+                             int in_dim, int out_dim, hipStream_t s);
+
 // gemv_mfma.hip, matmul_grouped_lora_down on the matrix cores: y[t *
 // y_stride + g * R + r] = sum_i W[g R + r, i] x[t * x_stride + g * D + i]
 // for a stacked Q4_K / Q6_K / Q8_0 matrix of G * R rows (device layout as

@@ -251,6 +251,36 @@ def test_moe_grouped_dsv4_formats(oracle, hip, n_tok):
     assert err <= MFMA_TOL
 
 
+@pytest.mark.parametrize("n_embd,n_ff,n_tok,k", [
+    (2048, 2048, 17, 1),   # one expert: a full batch and a batch of one slot
+    (4096, 2048, 41, 1),   # 16-slot batches and a remainder, two super-tiles of K
+    (2048, 4096, 70, 2),   # down over two super-tiles
+    (2304, 2048, 40, 1),   # 2304 rows of down (no whole number of row blocks), gate and up unstaged
+])
+def test_moe_16_slot_dsv4_formats(oracle, hip, n_embd, n_ff, n_tok, k):
+    """More than 8 slots an expert on average: IQ2_XXS gate/up and Q2_K down
+    in 16-slot batches staged through LDS, the Q2_K mins through sub-block
+    sums; one token far smaller and one with its signs aligned, so the sums
+    are large. (Not a far larger token: scaled by s its gate errors, about
+    1e-6 s in both sums' fp32, meet activations the clamp holds at 10, so
+    1e-4 of the output at s = 1e3 says nothing of the kernel.)"""
+    n_expert = 1 if n_tok == 17 else 2
+    gate, up, down, x, ids, w = make_case(n_tok, n_embd, n_ff, n_expert, k, G.IQ2_XXS, G.Q2_K,
+                                          820 + n_tok)
+    x[0] *= 1e-3
+    x[1] = np.abs(x[1])
+    w[2, 0] = 0.0  # a skipped slot
+    got = np.zeros(n_tok * n_embd, np.float32)
+    hip.moe_routed(got, x.reshape(-1), gate, up, down, ids, w, n_tok, n_embd, n_ff, n_expert, k,
+                   G.IQ2_XXS, G.Q2_K, 10.0)
+    toks = np.unique(np.array([0, 1, 2, n_tok // 2, n_tok - 1]))
+    want = run_oracle(oracle, np.zeros(len(toks) * n_embd, np.float32), x[toks], gate, up, down,
+                      ids[toks], w[toks], len(toks), n_embd, n_ff, n_expert, k, G.IQ2_XXS, G.Q2_K)
+    got, want = got.reshape(n_tok, n_embd)[toks], want.reshape(len(toks), n_embd)
+    for g, e in zip(got, want):
+        assert np.abs(g - e).max() <= MFMA_TOL * max(np.abs(e).max(), 1e-30)
+
+
 def test_moe_grouped_q6k_full_range_scales(oracle, hip):
     """Q6_K experts whose scales span the whole int8 range (sc (q - 32) up to
     4096, past f16's exact integers) on the grouped matrix-core route: the
