@@ -31,6 +31,25 @@ def test_weight_f32_f32_arm(oracle, hip, n_tok, in_dim, out_dim):
     assert err <= REL_TOL
 
 
+@pytest.mark.parametrize("n_tok,in_dim,out_dim", [
+    (1, 4096, 256),   # 16 wavefronts a row
+    (6, 4096, 256),   # the same, two passes of tokens
+    (1, 700, 257),    # two rows in one workgroup, three tiles, a ragged one
+    (5, 1030, 600),   # three rows a workgroup, splits of unequal length
+    (2, 513, 1),      # one row
+])
+def test_weight_f32_split_rows(oracle, hip, n_tok, in_dim, out_dim):
+    """Few rows per CU: each row's sum over several wavefronts, in fp32 like
+    the reference's (sums of in_dim terms: 2e-5 of the largest output)."""
+    w = f32_weights(out_dim, in_dim, in_dim + out_dim)
+    x = synth.activations(n_tok, in_dim, 4).reshape(-1)
+    rc, want = oracle.matmul_weight_f32(w, x, n_tok, in_dim, out_dim, oracle.F32)
+    assert rc == 0
+    got = np.full(n_tok * out_dim, np.nan, np.float32)
+    hip.matmul_weight_f32(got, w, x, n_tok, in_dim, out_dim, G.F32)
+    assert rel_err(got, want) <= 2e-5
+
+
 def test_weight_f32_hand_dot(hip):
     # weight.rs:329-354, exact in any summation order
     w = np.array([1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 1], np.float32)
