@@ -383,9 +383,9 @@ template <class F, int NW = 4, int ROWS = kMfsRows> struct MfsGeo {
 // the lo plane. NW wavefronts (64 NW threads) split each chunk's 8 steps,
 // 8 / NW each, for every row tile. smem: MfsGeo<F, NW, ROWS>::LDS bytes.
 // ROWX (NT = 1): a per-row image (a piece's hi and lo 16 bytes side by
-// side), the row of the lane's column (r16 & 7 packed, else r16) at byte
+// side), the row of the lane's column (r16 / 2 packed, else r16) at byte
 // xcol, and lanes 0..15 hold their column's unscale in usc (unscale
-// unused).
+// unused); packed, A row 2 t + plane holds a plane of token t.
 template <class F, int NT, bool PACK = false, int NW = 4, int ROWS = kMfsRows, bool ROWX = false>
 __device__ __forceinline__ void mfs_rows(const uint8_t *__restrict__ w,
                                          const _Float16 *__restrict__ xh, uint32_t plane_bytes,
@@ -452,7 +452,10 @@ __device__ __forceinline__ void mfs_rows(const uint8_t *__restrict__ w,
                     if (ROWX) {
                         const uint32_t o = xcol + (uint32_t)(((st * 4 + j) * 4 + q) * 32);
                         if (PACK) {
-                            xr[u][j][nt] = bload16(rx, o + (r16 >= 8 ? 16u : 0u), 0);
+                            // A row 2 t + plane: neighbouring lanes take
+                            // the hi and lo 16 bytes of one piece (half the
+                            // cache-line lookups of planes eight rows apart)
+                            xr[u][j][nt] = bload16(rx, o + 16u * (uint32_t)(r16 & 1), 0);
                         } else {
                             xr[u][j][nt] = bload16(rx, o, 0);
                             lr[u][j][nt] = bload16(rx, o + 16u, 0);
@@ -537,6 +540,21 @@ __device__ __forceinline__ void mfs_rows(const uint8_t *__restrict__ w,
         for (int i = 0; i < 4; i++) uq[i] = __shfl(usc, 4 * q + i, 64);
     }
     __syncthreads();
+    if constexpr (PACK && ROWX) {
+        // D rows 4 q + 0..3: the hi and lo sums of tokens 2 q and 2 q + 1
+        for (int e = tid; e < RT * 64; e += TH) {
+            const int rt = e / 64, ln = e % 64;
+            f32x4 v = red[rt * 64 + ln];
+#pragma unroll
+            for (int k = 1; k < NW; k++) v += red[(k * RT + rt) * 64 + ln];
+            const int o = row0 + 16 * rt + (ln & 15), t0 = 2 * (ln >> 4);
+            if (o < out_dim) {
+                if (t0 < n_tok) y[(size_t)t0 * y_stride + o] = (v[0] + v[1]) * uq[0];
+                if (t0 + 1 < n_tok) y[(size_t)(t0 + 1) * y_stride + o] = (v[2] + v[3]) * uq[2];
+            }
+        }
+        return;
+    }
     for (int e = tid; e < RT * NT * 64; e += TH) {
         const int rt = e / (NT * 64), nt = (e / 64) % NT, ln = e % 64;
         if (PACK && ln >= 32) continue;
@@ -971,7 +989,7 @@ __global__ __launch_bounds__(256) void k_gemv_mfl(const uint8_t *__restrict__ w,
                                        red, kMfgBatch);
 }
 
-// Batch column of lane r16 (c = r16 & 7 in the packed 8-column operand,
+// Batch column of lane r16 (c = r16 / 2 in the packed 8-column operand,
 // else r16; columns past the batch's count read its first column, whose
 // results are not stored) and its image row: the slot's token (tok given,
 // gate/up) or the slot (down); its byte offset in a plane and its unscale.
@@ -1042,7 +1060,7 @@ __global__ __launch_bounds__(PACK ? 64 * kMfsPackWaves : 256) void k_gemv_mfgs(c
     constexpr int bw = PACK ? 8 : kMfgBatch;
     uint32_t xcol;
     float usc;
-    mfg_column(bt, tok, unscale, in_dim, threadIdx.x & (bw - 1), xcol, usc);
+    mfg_column(bt, tok, unscale, in_dim, PACK ? (threadIdx.x & 15) >> 1 : threadIdx.x & 15, xcol, usc);
     mfs_rows<F, 1, PACK, PACK ? kMfsPackWaves : 4, ROWS, true>(
         w, xh, plane_bytes, nullptr, y, out_dim, bt.count, in_dim, out_dim,
         (int)blockIdx.x * ROWS, 0, in_dim / kMfsK, bw, smem, xcol, usc);
