@@ -58,6 +58,32 @@ constexpr int kQ8Chunk = 128;
 constexpr int kQ8Pad = kQ8Chunk + 1;  // LDS row stride (floats)
 constexpr int kQ8Tile = 272;          // 8 blocks: qs 8*32 | d 8*2
 
+// acc + pr[0] + pr[1] + ... + pr[n - 1], in that order; a whole chunk of N
+// reads 16 values ahead of the chain of adds, so it does not wait for LDS at
+// every one.
+template <int N>
+__device__ __forceinline__ float q8_sum(const float *pr, int n, float acc) {
+#pragma clang fp contract(off)
+    if (n < N) {
+        for (int i = 0; i < n; i++) acc = acc + pr[i];
+        return acc;
+    }
+    float v[16], u[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) v[i] = pr[i];
+#pragma unroll
+    for (int i0 = 0; i0 < N; i0 += 16) {
+        if (i0 + 16 < N)
+#pragma unroll
+            for (int i = 0; i < 16; i++) u[i] = pr[i0 + 16 + i];
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc = acc + v[i];
+#pragma unroll
+        for (int i = 0; i < 16; i++) v[i] = u[i];
+    }
+    return acc;
+}
+
 template <int ROWS, int BT>
 __global__ __launch_bounds__(256) void k_q8_int8_gemv(const uint8_t *__restrict__ w,
                                                       uint32_t w_bytes,
@@ -133,7 +159,7 @@ __global__ __launch_bounds__(256) void k_q8_int8_gemv(const uint8_t *__restrict_
         if (tid < BT * ROWS) {
             const float *pr = prod + tid * kQ8Pad;
             const int n = min(kQ8Chunk, blocks - c0);
-            for (int i = 0; i < n; i++) acc = acc + pr[i];
+            acc = q8_sum<kQ8Chunk>(pr, n, acc);
         }
         __syncthreads();
     }
@@ -236,7 +262,7 @@ __global__ __launch_bounds__(256) void k_q8_int8_rows(const uint8_t *__restrict_
         if (tid < BT * ROWS) {
             const float *pr = prod + tid * Pad;
             const int n = min(CB, blocks - c0);
-            for (int i = 0; i < n; i++) acc = acc + pr[i];
+            acc = q8_sum<CB>(pr, n, acc);
         }
         __syncthreads();
     }
