@@ -102,14 +102,113 @@ struct DevBuf {
     }
 };
 
+// Pinned host staging for the activations and outputs of the host-pointer
+// entry points. A small copy from or to pageable memory costs the runtime a
+// blocking round trip (4096 x 4096 Q4_K, one token, 16 KB each way: 33.8 us a
+// call); staged here both are plain asynchronous copies (27.7 us; the kernels
+// writing the pinned buffer themselves, 29.9: their stores cross the bus row by
+// row). See PinnedCopies.
+// Buffers of kPinBytes, one per thread that calls; a thread that ends returns
+// its buffer to the free list, so there are never more than threads that
+// called at the same time.
+constexpr size_t kPinBytes = (size_t)1 << 20;
+std::mutex g_pin_mu;
+// never destroyed (as g_scratch_map): the HIP runtime may be gone by then
+auto *g_pin_free = new std::vector<uint8_t *>();
+struct PinBuf {
+    uint8_t *p = nullptr;
+    uint8_t *get() {
+        if (p) return p;
+        {
+            std::lock_guard<std::mutex> lk(g_pin_mu);
+            if (!g_pin_free->empty()) {
+                p = g_pin_free->back();
+                g_pin_free->pop_back();
+                return p;
+            }
+        }
+        void *v = nullptr;
+        if (hipHostMalloc(&v, kPinBytes, hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;  // the copies go unstaged
+        }
+        return p = static_cast<uint8_t *>(v);
+    }
+    ~PinBuf() {
+        if (!p) return;
+        std::lock_guard<std::mutex> lk(g_pin_mu);
+        g_pin_free->push_back(p);
+    }
+};
+
 // Per calling thread: the stream and host<->device staging of the
 // host-pointer entry points (each such call synchronises before it returns).
 struct ThreadCtx {
     int device = -1;
     hipStream_t stream = nullptr;
     DevBuf w_raw, w_dev, x, y, moe_in, moe_w[3];
+    PinBuf pin;
 };
 thread_local ThreadCtx t_ctx;
+
+// One call's copies on the thread's stream, through the thread's pinned
+// buffer while they fit in it (a larger one goes straight to hipMemcpyAsync,
+// which pipelines its own staging). finish() synchronises and hands the
+// staged outputs over; a call that returns early on an error leaves its
+// copies to drain into the buffer, which wait() of the destructor sees to, so
+// the next call never shares it with them.
+class PinnedCopies {
+  public:
+    explicit PinnedCopies(ThreadCtx &c) : c_(c) {}
+    PinnedCopies(const PinnedCopies &) = delete;
+    ~PinnedCopies() {
+        if (used_ && !finished_) (void)hipStreamSynchronize(c_.stream);
+    }
+    hipError_t to_device(void *dst, const void *src, size_t n) {
+        if (n == 0) return hipSuccess;
+        if (uint8_t *b = take(n)) {
+            std::memcpy(b, src, n);
+            src = b;
+        }
+        return hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, c_.stream);
+    }
+    hipError_t to_host(void *dst, const void *src, size_t n) {
+        if (n == 0) return hipSuccess;
+        if (uint8_t *b = n_out_ < kMaxOut ? take(n) : nullptr) {
+            out_[n_out_++] = {dst, b, n};
+            dst = b;
+        }
+        return hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, c_.stream);
+    }
+    hipError_t finish() {
+        const hipError_t e = hipStreamSynchronize(c_.stream);
+        finished_ = true;
+        if (e == hipSuccess)
+            for (int i = 0; i < n_out_; i++) std::memcpy(out_[i].dst, out_[i].src, out_[i].n);
+        return e;
+    }
+
+  private:
+    struct Out {
+        void *dst;
+        const uint8_t *src;
+        size_t n;
+    };
+    static constexpr int kMaxOut = 4;
+    uint8_t *take(size_t n) {
+        if (n > kPinBytes - used_) return nullptr;
+        uint8_t *b = c_.pin.get();
+        if (!b) return nullptr;
+        b += used_;
+        used_ = std::min(kPinBytes, used_ + (n + 255) / 256 * 256);
+        return b;
+    }
+    ThreadCtx &c_;
+    Out out_[kMaxOut];
+    int n_out_ = 0;
+    size_t used_ = 0;
+    bool finished_ = false;
+};
 
 // Device workspace of the kernels (activation images, MoE tables and
 // intermediates), one set per (device, stream). Work on one stream runs in
@@ -773,6 +872,7 @@ int rsllm_hip_matmul_quant_f32(float *out, size_t out_len, const uint8_t *weight
     }
     if ((rc = ensure_device())) return rc;
     ThreadCtx &c = t_ctx;
+    PinnedCopies io(c);
     const Lease reg = find_registered(weights, weights_len, dtype, in_dim);
     const uint8_t *dw = reg.dev;
     if (!dw) {
@@ -789,16 +889,14 @@ int rsllm_hip_matmul_quant_f32(float *out, size_t out_len, const uint8_t *weight
     }
     HIP_TRY(c.x.ensure(x_len * sizeof(float)), "hipMalloc");
     HIP_TRY(c.y.ensure(out_len * sizeof(float)), "hipMalloc");
-    HIP_TRY(hipMemcpyAsync(c.x.p, x, x_len * sizeof(float), hipMemcpyHostToDevice, c.stream),
-            "upload x");
+    HIP_TRY(io.to_device(c.x.p, x, x_len * sizeof(float)), "upload x");
     ScratchLease sc = stream_scratch(c.stream);
     HIP_TRY(sc->xq.ensure(gemv_work_bytes(dtype, (int)n_tok, (int)in_dim, (int)out_dim)), "hipMalloc");
     HIP_TRY(launch_gemv(dtype, dw, weights_len, (const float *)c.x.p, (uint8_t *)sc->xq.p,
                         (float *)c.y.p, (int)n_tok, (int)in_dim, (int)out_dim, c.stream),
             "gemv");
-    HIP_TRY(hipMemcpyAsync(out, c.y.p, out_len * sizeof(float), hipMemcpyDeviceToHost, c.stream),
-            "download out");
-    HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
+    HIP_TRY(io.to_host(out, c.y.p, out_len * sizeof(float)), "download out");
+    HIP_TRY(io.finish(), "hipStreamSynchronize");
     return ok();
 }
 
@@ -981,6 +1079,7 @@ int rsllm_hip_moe_routed(float *out, size_t out_len, const float *x, size_t x_le
     if (n_tok == 0 || k == 0) return ok();
     if ((rc = ensure_device())) return rc;
     ThreadCtx &c = t_ctx;
+    PinnedCopies io(c);
     // expert blobs: registered device copies, else uploaded (and converted to
     // the device layout) for this call
     const uint8_t *blob[3] = {gate, up, down};
@@ -1000,11 +1099,10 @@ int rsllm_hip_moe_routed(float *out, size_t out_len, const float *x, size_t x_le
     float *d_x = (float *)base, *d_out = (float *)(base + a_x);
     int32_t *d_ids = (int32_t *)(base + a_x + a_o);
     float *d_w = (float *)(base + a_x + a_o + a_i);
-    HIP_TRY(hipMemcpyAsync(d_x, x, x_len * 4, hipMemcpyHostToDevice, c.stream), "upload x");
-    HIP_TRY(hipMemcpyAsync(d_out, out, out_len * 4, hipMemcpyHostToDevice, c.stream), "upload out");
-    HIP_TRY(hipMemcpyAsync(d_ids, ids, ids_len * 4, hipMemcpyHostToDevice, c.stream), "upload ids");
-    HIP_TRY(hipMemcpyAsync(d_w, weights, ids_len * 4, hipMemcpyHostToDevice, c.stream),
-            "upload weights");
+    HIP_TRY(io.to_device(d_x, x, x_len * 4), "upload x");
+    HIP_TRY(io.to_device(d_out, out, out_len * 4), "upload out");
+    HIP_TRY(io.to_device(d_ids, ids, ids_len * 4), "upload ids");
+    HIP_TRY(io.to_device(d_w, weights, ids_len * 4), "upload weights");
     ScratchLease sc = stream_scratch(c.stream);
     HIP_TRY(sc->moe.ensure(moe_scratch_bytes(dtype_gate_up, dtype_down, (int)n_tok, (int)k,
                                              (int)n_expert, (int)n_embd, (int)n_ff)),
@@ -1013,9 +1111,8 @@ int rsllm_hip_moe_routed(float *out, size_t out_len, const float *x, size_t x_le
                        down_len / n_expert, d_x, d_ids, d_w, d_out, (uint8_t *)sc->moe.p,
                        (int)n_tok, (int)k, (int)n_expert, (int)n_embd, (int)n_ff, clamp, c.stream),
             "moe");
-    HIP_TRY(hipMemcpyAsync(out, d_out, out_len * 4, hipMemcpyDeviceToHost, c.stream),
-            "download out");
-    HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
+    HIP_TRY(io.to_host(out, d_out, out_len * 4), "download out");
+    HIP_TRY(io.finish(), "hipStreamSynchronize");
     return ok();
 }
 
@@ -1092,6 +1189,7 @@ int rsllm_hip_quantize_q8_0_batch(const float *x, size_t x_len, int8_t *xq, size
     if (n_tok == 0) return ok();
     if ((rc = ensure_device())) return rc;
     ThreadCtx &c = t_ctx;
+    PinnedCopies io(c);
     const size_t a_x = (x_len * 4 + 255) / 256 * 256, a_q = (xq_len + 255) / 256 * 256;
     const size_t a_s = (scale_len * 4 + 255) / 256 * 256;
     HIP_TRY(c.x.ensure(a_x + a_q + a_s + 256), "hipMalloc");
@@ -1100,16 +1198,15 @@ int rsllm_hip_quantize_q8_0_batch(const float *x, size_t x_len, int8_t *xq, size
     int8_t *d_q = (int8_t *)(base + a_x);
     float *d_s = (float *)(base + a_x + a_q);
     int32_t *d_st = (int32_t *)(base + a_x + a_q + a_s);
-    HIP_TRY(hipMemcpyAsync(d_x, x, x_len * 4, hipMemcpyHostToDevice, c.stream), "upload x");
+    HIP_TRY(io.to_device(d_x, x, x_len * 4), "upload x");
     HIP_TRY(launch_fill_zero(reinterpret_cast<float *>(d_st), 1, c.stream), "fill_zero");
     HIP_TRY(launch_q8_quantize(d_x, d_q, d_s, (int)n_tok, (int)in_dim, d_st, c.stream),
             "q8_quantize");
     int32_t st = 0;
-    HIP_TRY(hipMemcpyAsync(xq, d_q, xq_len, hipMemcpyDeviceToHost, c.stream), "download xq");
-    HIP_TRY(hipMemcpyAsync(scale, d_s, scale_len * 4, hipMemcpyDeviceToHost, c.stream),
-            "download scale");
-    HIP_TRY(hipMemcpyAsync(&st, d_st, 4, hipMemcpyDeviceToHost, c.stream), "download status");
-    HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
+    HIP_TRY(io.to_host(xq, d_q, xq_len), "download xq");
+    HIP_TRY(io.to_host(scale, d_s, scale_len * 4), "download scale");
+    HIP_TRY(io.to_host(&st, d_st, 4), "download status");
+    HIP_TRY(io.finish(), "hipStreamSynchronize");
     if (st)
         return set_err(RSLLM_HIP_ERR_NON_FINITE_INPUT, "quantize_q8_0: activation");
     return ok();
@@ -1153,6 +1250,7 @@ int rsllm_hip_matmul_q8_0_batch(float *out, size_t out_len, const uint8_t *weigh
     }
     if ((rc = ensure_device())) return rc;
     ThreadCtx &c = t_ctx;
+    PinnedCopies io(c);
     // device layout: a registered copy (Q8_0 with this in_dim), else the rows
     // uploaded and regrouped for this call
     const Lease reg = find_registered(weights, weights_len, T_Q8_0, in_dim);
@@ -1171,17 +1269,15 @@ int rsllm_hip_matmul_q8_0_batch(float *out, size_t out_len, const uint8_t *weigh
     HIP_TRY(c.x.ensure(a_q + xscale_len * 4), "hipMalloc");
     int8_t *d_q = (int8_t *)c.x.p;
     float *d_s = (float *)((uint8_t *)c.x.p + a_q);
-    HIP_TRY(hipMemcpyAsync(d_q, xq, xq_len, hipMemcpyHostToDevice, c.stream), "upload xq");
-    HIP_TRY(hipMemcpyAsync(d_s, xscale, xscale_len * 4, hipMemcpyHostToDevice, c.stream),
-            "upload xscale");
+    HIP_TRY(io.to_device(d_q, xq, xq_len), "upload xq");
+    HIP_TRY(io.to_device(d_s, xscale, xscale_len * 4), "upload xscale");
     HIP_TRY(c.y.ensure(out_len * sizeof(float)), "hipMalloc");
     HIP_TRY(launch_q8_int8_matmul(dw, weights_len, d_q, d_s,
                                   (float *)c.y.p, (int)n_tok, (int)in_dim, (int)out_dim,
                                   c.stream),
             "q8_matmul");
-    HIP_TRY(hipMemcpyAsync(out, c.y.p, out_len * sizeof(float), hipMemcpyDeviceToHost, c.stream),
-            "download out");
-    HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
+    HIP_TRY(io.to_host(out, c.y.p, out_len * sizeof(float)), "download out");
+    HIP_TRY(io.finish(), "hipStreamSynchronize");
     return ok();
 }
 
@@ -1286,14 +1382,14 @@ int rsllm_hip_dequant_to_f32(uint32_t dtype, const uint8_t *src, size_t src_len,
     if (dst_len == 0) return ok();
     if ((rc = ensure_device())) return rc;
     ThreadCtx &c = t_ctx;
+    PinnedCopies io(c);
     HIP_TRY(c.w_raw.ensure(src_len), "hipMalloc");
     HIP_TRY(c.y.ensure(dst_len * sizeof(float)), "hipMalloc");
-    HIP_TRY(hipMemcpyAsync(c.w_raw.p, src, src_len, hipMemcpyHostToDevice, c.stream), "upload");
+    HIP_TRY(io.to_device(c.w_raw.p, src, src_len), "upload");
     HIP_TRY(launch_dequant(dtype, (const uint8_t *)c.w_raw.p, (float *)c.y.p, dst_len, c.stream),
             "dequant");
-    HIP_TRY(hipMemcpyAsync(dst, c.y.p, dst_len * sizeof(float), hipMemcpyDeviceToHost, c.stream),
-            "download");
-    HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
+    HIP_TRY(io.to_host(dst, c.y.p, dst_len * sizeof(float)), "download");
+    HIP_TRY(io.finish(), "hipStreamSynchronize");
     return ok();
 }
 
@@ -1321,6 +1417,7 @@ int rsllm_hip_matmul_weight_f32(float *out, size_t out_len, const uint8_t *weigh
     if (n_tok == 0 || out_dim == 0) return ok();
     if ((rc = ensure_device())) return rc;
     ThreadCtx &c = t_ctx;
+    PinnedCopies io(c);
     const Lease reg = find_registered(weights, weights_len, dtype, in_dim);
     const uint8_t *dw = reg.dev;
     if (!dw && weights_len) {
@@ -1338,15 +1435,13 @@ int rsllm_hip_matmul_weight_f32(float *out, size_t out_len, const uint8_t *weigh
     HIP_TRY(c.x.ensure(x_len * sizeof(float) + 16), "hipMalloc");
     HIP_TRY(c.y.ensure(out_len * sizeof(float)), "hipMalloc");
     if (x_len)
-        HIP_TRY(hipMemcpyAsync(c.x.p, x, x_len * sizeof(float), hipMemcpyHostToDevice, c.stream),
-                "upload x");
+        HIP_TRY(io.to_device(c.x.p, x, x_len * sizeof(float)), "upload x");
     ScratchLease sc = stream_scratch(c.stream);
     rc = weight_f32_compute((float *)c.y.p, out_len, dw, weights_len, (const float *)c.x.p, n_tok,
                             in_dim, out_dim, dtype, c.stream, *sc);
     if (rc) return rc;
-    HIP_TRY(hipMemcpyAsync(out, c.y.p, out_len * sizeof(float), hipMemcpyDeviceToHost, c.stream),
-            "download out");
-    HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
+    HIP_TRY(io.to_host(out, c.y.p, out_len * sizeof(float)), "download out");
+    HIP_TRY(io.finish(), "hipStreamSynchronize");
     return ok();
 }
 
@@ -1376,6 +1471,7 @@ int rsllm_hip_matmul_grouped_lora_down(float *out, size_t out_len, const uint8_t
     if (n_tok == 0 || n_groups == 0 || rank == 0) return ok();
     if ((rc = ensure_device())) return rc;
     ThreadCtx &c = t_ctx;
+    PinnedCopies io(c);
     // The blob may be longer; the groups use this much. The device layout
     // packs 8 blocks per super-tile with a shorter last one, so a group's
     // slice of the whole matrix's layout is the group's own layout only when
@@ -1415,15 +1511,13 @@ int rsllm_hip_matmul_grouped_lora_down(float *out, size_t out_len, const uint8_t
     HIP_TRY(c.x.ensure(x_len * sizeof(float) + 16), "hipMalloc");
     HIP_TRY(c.y.ensure(out_len * sizeof(float)), "hipMalloc");
     if (x_len)
-        HIP_TRY(hipMemcpyAsync(c.x.p, x, x_len * sizeof(float), hipMemcpyHostToDevice, c.stream),
-                "upload x");
+        HIP_TRY(io.to_device(c.x.p, x, x_len * sizeof(float)), "upload x");
     ScratchLease sc = stream_scratch(c.stream);
     rc = lora_down_compute((float *)c.y.p, out_len, dw, stride, (const float *)c.x.p, n_tok,
                            n_groups, group_dim, rank, dtype, c.stream, *sc, per_group);
     if (rc) return rc;
-    HIP_TRY(hipMemcpyAsync(out, c.y.p, out_len * sizeof(float), hipMemcpyDeviceToHost, c.stream),
-            "download out");
-    HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
+    HIP_TRY(io.to_host(out, c.y.p, out_len * sizeof(float)), "download out");
+    HIP_TRY(io.finish(), "hipStreamSynchronize");
     return ok();
 }
 
@@ -1455,6 +1549,7 @@ int rsllm_hip_apply_shared_expert(float *out, size_t out_len, const float *x, si
     if (n_tok == 0 || n_embd == 0) return ok();
     if ((rc = ensure_device())) return rc;
     ThreadCtx &c = t_ctx;
+    PinnedCopies io(c);
     const uint8_t *blob[3] = {gate, up, down};
     const size_t blen[3] = {gate_len, up_len, down_len};
     const uint32_t bdt[3] = {dtype_gate, dtype_up, dtype_down};
@@ -1466,16 +1561,14 @@ int rsllm_hip_apply_shared_expert(float *out, size_t out_len, const float *x, si
             return rc;
     HIP_TRY(c.x.ensure(x_len * sizeof(float) + 16), "hipMalloc");
     HIP_TRY(c.y.ensure(out_len * sizeof(float)), "hipMalloc");
-    HIP_TRY(hipMemcpyAsync(c.x.p, x, x_len * sizeof(float), hipMemcpyHostToDevice, c.stream),
-            "upload x");
+    HIP_TRY(io.to_device(c.x.p, x, x_len * sizeof(float)), "upload x");
     ScratchLease sc = stream_scratch(c.stream);
     rc = shared_compute((float *)c.y.p, (const float *)c.x.p, dev[0], gate_len, dtype_gate, dev[1],
                         up_len, dtype_up, dev[2], down_len, dtype_down, n_tok, n_embd, n_ff, clamp,
                         c.stream, *sc);
     if (rc) return rc;
-    HIP_TRY(hipMemcpyAsync(out, c.y.p, out_len * sizeof(float), hipMemcpyDeviceToHost, c.stream),
-            "download out");
-    HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
+    HIP_TRY(io.to_host(out, c.y.p, out_len * sizeof(float)), "download out");
+    HIP_TRY(io.finish(), "hipStreamSynchronize");
     return ok();
 }
 
