@@ -21,9 +21,10 @@
 // eight times: 4.4 GB from memory for 1.1 GB of weights.)
 //
 // DS-V4 experts (256 x IQ2_XXS gate/up 2048 x 4096, Q2_K down 4096 x 2048,
-// top-6) at 512 tokens: gate/up 803 us, down 363 us, the call 1153 us, against
-// 941, 482 and 1480 us on mf_rows. Gate/up is bound by the vector work of the
-// decode (about 93 instructions per 16 x 128 weights) and its table reads.
+// top-6) at 512 tokens: the call 1062 us, against 1480 us on mf_rows (1143 us
+// before the IQ2_XXS steps were staggered and the loop freed of spilled
+// addresses). Gate/up is bound by the vector work of the decode (about 97
+// instructions per 16 x 128 weights) and its table reads.
 #include "mfma_formats.h"
 #include "buffer_lds.h"
 
@@ -34,6 +35,7 @@ namespace rsllm_hip {
 constexpr int kXmCopies = 16;
 constexpr int kXmTables = (256 + 128) * kXmCopies * 16;
 __device__ __forceinline__ void xm_stage_tables(uint4 *tab, int threads) {
+#pragma unroll 2
     for (int i = threadIdx.x; i < 384 * kXmCopies; i += threads) {
         const int e = i / kXmCopies;
         tab[i] = e < 256 ? *reinterpret_cast<const uint4 *>(kIq2F16.grid[e])
@@ -71,32 +73,71 @@ template <> struct XmFmt<MIQ2> {
     __device__ void put(uint8_t *buf, int lane, int b) const {
         *reinterpret_cast<uint4 *>(buf + (lane >> 2) * kXmRow + 16 * (lane & 3)) = qs[b];
     }
-    // the sub-group scales differ within a step: each MFMA result is scaled
-    // here (as MIQ2::step)
-    __device__ void step(const uint8_t *buf, int r16, int q, int b, int h, const uint4 (&x)[4],
-                         const uint4 (&xl)[4], f32x4 &, f32x4 &acc, const uint8_t *tab) const {
-        const uint8_t *r = buf + r16 * kXmRow + 32 * h;
-        const uint4 a0 = *reinterpret_cast<const uint4 *>(r), a1 = *reinterpret_cast<const uint4 *>(r + 16);
-        const float dv = f16_to_f32(((b & 2) ? d.y : d.x) >> (16 * (b & 1)) & 0xFFFFu);
-        const float d4 = dv * 0.25f, d8 = dv * 0.125f;
+    // The sub-group scales differ within a step, so each MFMA result is scaled
+    // (as MIQ2::step) into P, the block's sum, which joins acc at its end: a
+    // chain of 8 and one of in_dim / 256 terms, whose rounding error is that
+    // of a K split over four wavefronts. Row tiles go through in units of two
+    // MFMA operands, staggered by hand: the records of unit u + 2 and the table
+    // entries of u + 1 are read, then u is multiplied and u - 1 scaled. (Left
+    // to the compiler every table read and every MFMA was waited for at once.)
+    template <int RT>
+    __device__ static void step_all(const XmFmt (&w)[RT], const uint8_t *buf, int r16, int q, int b, int h,
+                                    const uint4 (&x)[4], const uint4 (&xl)[4], f32x4 (&P)[RT],
+                                    f32x4 (&acc)[RT], const uint8_t *tab) {
+        constexpr int U = 2 * RT;
+        uint4 a[U], gv[U][2], sv[U][2];
+        f32x4 S[U][2];
+        auto record = [&](int u) {
+            a[u] = *reinterpret_cast<const uint4 *>(buf + (u >> 1) * kBuf + r16 * kXmRow + 32 * h + 16 * (u & 1));
+        };
+        auto gather = [&](int u) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const uint4 &a = j < 2 ? a0 : a1;
-            const uint32_t aux0 = (j & 1) ? a.z : a.x, aux1 = (j & 1) ? a.w : a.y;
-            const float db = fmaf((float)(aux1 >> 28), d4, d8);
-            const uint4 gv = *reinterpret_cast<const uint4 *>(
-                tab + ((aux0 >> (8 * q)) & 0xFFu) * (16 * kXmCopies));
-            const uint4 sv = *reinterpret_cast<const uint4 *>(
-                tab + 256 * 16 * kXmCopies + ((aux1 >> (7 * q)) & 0x7Fu) * (16 * kXmCopies));
-            const f16x8 bv = __builtin_bit_cast(
-                f16x8, make_uint4(gv.x ^ sv.x, gv.y ^ sv.y, gv.z ^ sv.z, gv.w ^ sv.w));
-            const f32x4 P0 = mfma16x32(x[j], bv, f32x4{0.f, 0.f, 0.f, 0.f});
-            const f32x4 P = mfma16x32(xl[j], bv, P0);
+            for (int k = 0; k < 2; k++) {
+                const uint32_t aux0 = k ? a[u].z : a[u].x, aux1 = k ? a[u].w : a[u].y;
+                gv[u][k] = *reinterpret_cast<const uint4 *>(tab + ((aux0 >> (8 * q)) & 0xFFu) * (16 * kXmCopies));
+                sv[u][k] = *reinterpret_cast<const uint4 *>(tab + 256 * 16 * kXmCopies +
+                                                            ((aux1 >> (7 * q)) & 0x7Fu) * (16 * kXmCopies));
+            }
+        };
+        auto multiply = [&](int u) {
+            f16x8 bv[2];
 #pragma unroll
-            for (int i = 0; i < 4; i++) acc[i] = fmaf(db, P[i], acc[i]);
+            for (int k = 0; k < 2; k++) {
+                const uint4 &g = gv[u][k], &s = sv[u][k];
+                bv[k] = __builtin_bit_cast(f16x8, make_uint4(g.x ^ s.x, g.y ^ s.y, g.z ^ s.z, g.w ^ s.w));
+            }
+#pragma unroll
+            for (int k = 0; k < 2; k++) S[u][k] = mfma16x32(x[2 * (u & 1) + k], bv[k], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int k = 0; k < 2; k++) S[u][k] = mfma16x32(xl[2 * (u & 1) + k], bv[k], S[u][k]);
+        };
+        auto scale = [&](int u) {
+            const int rt = u >> 1;
+            const float dv = f16_to_f32(((b & 2) ? w[rt].d.y : w[rt].d.x) >> (16 * (b & 1)) & 0xFFFFu);
+            const float d4 = dv * 0.25f, d8 = dv * 0.125f;
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const float db = fmaf((float)((k ? a[u].w : a[u].y) >> 28), d4, d8);
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    P[rt][i] = h || (u & 1) || k ? fmaf(db, S[u][k][i], P[rt][i]) : db * S[u][k][i];
+            }
+            if (h && (u & 1)) acc[rt] += P[rt];
+        };
+        record(0);
+        record(1);
+        gather(0);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (u + 2 < U) record(u + 2);
+            if (u + 1 < U) gather(u + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(u);
+            if (u > 0) scale(u - 1);
+            __builtin_amdgcn_sched_barrier(0);
         }
+        scale(U - 1);
     }
-    __device__ void fold(const uint8_t *, int, int, int, const uint4 &, f32x4 &, f32x4 &) const {}
 };
 // Q2_K: w = d sc q - dmin m per 16-element sub-block. B = 2^-15 sc q: a qs
 // byte zero-extended to 16 bits and masked to code j is the f16 subnormal q
@@ -167,7 +208,7 @@ template <> struct XmFmt<MQ2K> {
         const uint32_t dv = sel4(dd, b);
         const float d = f16_to_f32(dv & 0xFFFFu) * 32768.0f, dmin = f16_to_f32(dv >> 16) * 16777216.0f;
 #pragma unroll
-        for (int i = 0; i < 4; i++) acc[i] = fmaf(-dmin, M[i], fmaf(d, P[i], acc[i]));
+        for (int i = 0; i < 4; i++) acc[i] += fmaf(-dmin, M[i], d * P[i]);
         P = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 };
@@ -229,33 +270,33 @@ __global__ __launch_bounds__(64 * kXmNW) void k_xm(const uint8_t *__restrict__ w
     uint32_t so = 0;
     if constexpr (G::SN != 0)
         so = image_row(2 * wv + ((lane >> 4) & 1)) * (uint32_t)(in_dim >> 2) + 16u * (uint32_t)(lane & 15);
-    auto dma_x = [&](int s) {
+    // slot: byte offset of step s's place in the ring, X (s % 3)
+    auto dma_x = [&](int s, uint32_t slot) {
         const bl_rsrc r = {rx[0], rx[1], s < ns ? rx[2] : 0u, rx[3]};
-        bl_dma16(r, xo, 512u * (uint32_t)s, lds_x + (uint32_t)(s % 3) * (uint32_t)G::X + 1024u * (uint32_t)wv);
+        bl_dma16(r, xo, 512u * (uint32_t)s, lds_x + slot + 1024u * (uint32_t)wv);
     };
     auto dma_s = [&](int hb) {
         const bl_rsrc r = {rsum[0], rsum[1], hb < nh ? rsum[2] : 0u, rsum[3]};
         if (lane < 32) bl_dma16(r, so, 256u * (uint32_t)hb, lds_s + (uint32_t)(hb & 1) * 4096u + 512u * (uint32_t)wv);
     };
-    uint32_t rp[RT], rr[RT];
-#pragma unroll
-    for (int rt = 0; rt < RT; rt++) {
-        rp[rt] = (uint32_t)min(row0 + 16 * rt + (lane >> 2), out_dim - 1) * X::row_bytes(in_dim) + 16u * (uint32_t)(lane & 3);
-        rr[rt] = (uint32_t)min(row0 + 16 * rt + r16, out_dim - 1) * X::row_bytes(in_dim);
-    }
+    // row tile rt's first row (uniform; a tile past the end repeats the last
+    // rows, a tile across it starts early), and the lane's place in a tile
+    auto tile_row = [&](int rt) { return max(min(row0 + 16 * rt, out_dim - 16), 0); };
+    const uint32_t rp = (uint32_t)min(lane >> 2, out_dim - 1) * X::row_bytes(in_dim) + 16u * (uint32_t)(lane & 3);
+    const uint32_t rr = (uint32_t)min(r16, out_dim - 1) * X::row_bytes(in_dim);
     X wc[RT];
     // blocks 2 p, 2 p + 1 of half hb, with p = 0 also what serves the half
     auto load_w = [&](int hb, int p) {
         const __amdgpu_buffer_rsrc_t r = hb < nh ? rw : make_rsrc(w0, 0);
-        const uint32_t so = (uint32_t)(hb >> 1) * X::kTile;
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
-            wc[rt].load(r, rp[rt], so, hb & 1, p);
-            if (p == 0) wc[rt].load_aux(r, rp[rt], rr[rt], so, hb & 1);
+            const uint32_t so = (uint32_t)tile_row(rt) * X::row_bytes(in_dim) + (uint32_t)(hb >> 1) * X::kTile;
+            wc[rt].load(r, rp, so, hb & 1, p);
+            if (p == 0) wc[rt].load_aux(r, rp, rr, so, hb & 1);
         }
     };
-    dma_x(0);
-    dma_x(1);
+    dma_x(0, 0);
+    dma_x(1, (uint32_t)G::X);
     if constexpr (G::SN != 0) dma_s(0);
     load_w(0, 0);
     load_w(0, 1);
@@ -273,6 +314,14 @@ __global__ __launch_bounds__(64 * kXmNW) void k_xm(const uint8_t *__restrict__ w
     for (int j = 0; j < 2; j++)
 #pragma unroll
         for (int l = 0; l < 2; l++) xa[j][l] = 512u * (uint32_t)r16 + 16u * (uint32_t)((8 * j + 2 * q + l) ^ r16);
+    // The compiler is kept from seeing through these offsets and the ring's:
+    // it would hold every step's sum of them in registers for the whole loop
+    // (50 spilled to scratch, reloaded with full waits once a half).
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int l = 0; l < 2; l++) asm("" : "+v"(xa[j][l]));
+    uint32_t slot = 0;
     // step i of half hb
     auto step = [&](int hb, auto i_c) __attribute__((always_inline)) {
         constexpr int i = decltype(i_c)::value, b = i >> 1, h = i & 1;
@@ -284,7 +333,8 @@ __global__ __launch_bounds__(64 * kXmNW) void k_xm(const uint8_t *__restrict__ w
         // step 7, when their registers are free)
         constexpr int kA = RT * (2 + X::kAux) + G::SN, kB = RT * 2;
         bl_barrier<1 + (i == 5 || i == 6 ? kA : i == 0 || i == 1 ? kB : 0)>();
-        dma_x(s + 2);
+        slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)slot);
+        dma_x(s + 2, slot == 0 ? 2u * (uint32_t)G::X : slot - (uint32_t)G::X);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (i == 4) {
             if constexpr (G::SN != 0) dma_s(hb + 1);
@@ -298,7 +348,8 @@ __global__ __launch_bounds__(64 * kXmNW) void k_xm(const uint8_t *__restrict__ w
         if constexpr (h == 0)
 #pragma unroll
             for (int rt = 0; rt < RT; rt++) wc[rt].put(wbuf + rt * X::kBuf, lane, b);
-        const uint8_t *xs = xbuf + (s % 3) * G::X;
+        const uint8_t *xs = xbuf + slot;
+        slot = slot == 2u * (uint32_t)G::X ? 0u : slot + (uint32_t)G::X;
         uint4 xr[4], xl[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -308,6 +359,13 @@ __global__ __launch_bounds__(64 * kXmNW) void k_xm(const uint8_t *__restrict__ w
         uint4 sm = make_uint4(0, 0, 0, 0);
         if constexpr (h == 1 && G::SN != 0)
             sm = *reinterpret_cast<const uint4 *>(sbuf + 4096 * (hb & 1) + 256 * r16 + 64 * b + 16 * q);
+        if constexpr (X::kTables) {
+            X::step_all(wc, wbuf, r16, q, b, h, xr, xl, P, acc, tab);
+            if constexpr (i == 7)
+#pragma unroll
+                for (int rt = 0; rt < RT; rt++) wc[rt].next();
+            return;
+        } else
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
             const uint8_t *buf = wbuf + rt * X::kBuf;
@@ -334,8 +392,8 @@ __global__ __launch_bounds__(64 * kXmNW) void k_xm(const uint8_t *__restrict__ w
     for (int i = 0; i < 4; i++) us[i] = unscale[image_row(4 * q + i)];
 #pragma unroll
     for (int rt = 0; rt < RT; rt++) {
-        const int o = row0 + 16 * rt + r16;
-        if (o >= out_dim) continue;
+        const int o = tile_row(rt) + r16;
+        if (row0 + 16 * rt >= out_dim || o >= out_dim) continue;
 #pragma unroll
         for (int i = 0; i < 4; i++)
             if (4 * q + i < bt.count) y[(size_t)(4 * q + i) * out_dim + o] = acc[rt][i] * us[i];
