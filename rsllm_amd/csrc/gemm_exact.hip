@@ -1,5 +1,5 @@
 // Matrix-core GEMM with exact weights for many tokens: y[t, o] = sum_i
-// W[o, i] x[t, i] where each 16-row weight tile is decoded once for up to 64
+// W[o, i] x[t, i] where each 16-row weight tile is decoded once for up to 48
 // token columns. The weights are the exact f16 integers of mfma_formats.h
 // with their fp32 scales, the activations hi + lo f16 planes (about 2^-22
 // relative), as in the batched GEMV (gemv_mfma.hip), whose 16- and 32-token
@@ -206,14 +206,27 @@ __global__ __launch_bounds__(64 * kXgWaves) void k_xg(const uint8_t *__restrict_
                 d[rt] = raw[rt].scale(u, KG);
             }
         };
-        auto fold = [&]() {
+        // A tile's sum, added to acc at its end: chains of 4 and of in_dim /
+        // 256 terms round like a K split over four wavefronts (in_dim 4096:
+        // error against 64 bits 1.2e-7, one chain 1.6e-7, the
+        // 16-token passes 1.3e-7).
+        f32x4 part[RT][NT];
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) part[rt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        auto fold = [&](int u) {
 #pragma unroll
             for (int nt = 0; nt < NT; nt++)
 #pragma unroll
                 for (int rt = 0; rt < RT; rt++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        acc[rt][nt][i] = fmaf(d[rt], P[nt][rt][i], acc[rt][nt][i]);
+                    for (int i = 0; i < 4; i++) {
+                        const float v = u == 0 ? d[rt] * P[nt][rt][i]
+                                               : fmaf(d[rt], P[nt][rt][i], part[rt][nt][i]);
+                        if (u == 3) acc[rt][nt][i] += v;
+                        else part[rt][nt][i] = v;
+                    }
         };
         auto mfmas = [&](int u) {
             uint4 hi = hi0, lo = lo0;
@@ -242,11 +255,11 @@ __global__ __launch_bounds__(64 * kXgWaves) void k_xg(const uint8_t *__restrict_
                 mfmas(u);
                 __builtin_amdgcn_sched_barrier(0);
                 read_x((u + 1) & 3, 0, hi0, lo0);
-                fold();
+                fold(u);
                 decode((u + 1) & 3);
             } else {
                 read_x(u, 0, hi0, lo0);
-                fold();
+                fold((u + 3) & 3);
                 decode(u);
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (u == 3) load_raw();
@@ -272,7 +285,7 @@ __global__ __launch_bounds__(64 * kXgWaves) void k_xg(const uint8_t *__restrict_
             step(4 * t + 2, std::integral_constant<int, 2>{});
             step(4 * t + 3, std::integral_constant<int, 3>{});
         }
-        if constexpr (KG == 1) fold();
+        if constexpr (KG == 1) fold(3);
     };
 
     dma_w(0);
@@ -379,7 +392,10 @@ static hipError_t xg_go(const uint8_t *w, const _Float16 *xh, const float *us, f
 
 // Column tiles per workgroup: the fewest (rounds of one workgroup per CU) x
 // (work of one), counting one column tile's time for what a workgroup does
-// whatever its width.
+// whatever its width. Four do not fit the registers beside the tile sums (65
+// spilled); with one chain of sums instead they served 16 x [512 x 1024] at
+// 400 tokens in 34 us (three: 42 us, the 16-token passes 76 us) at an error
+// above the passes' own (1.1e-7 against 9.9e-8; now 9.6e-8).
 template <class F>
 static hipError_t xg_launch(const uint8_t *w, const float *x, uint8_t *scratch, float *y,
                             const XgShape &sh, hipStream_t s) {
@@ -390,9 +406,9 @@ static hipError_t xg_launch(const uint8_t *w, const float *x, uint8_t *scratch, 
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const long cus = device_cus();
-    int best = 4;
+    int best = 3;
     long cost = -1;
-    for (int nt = 4; nt >= 2; nt--) {
+    for (int nt = 3; nt >= 2; nt--) {
         const long tiles = (long)sh.groups * ((sh.group_rows + 255) / 256) *
                            ((sh.n_cols + 16 * nt - 1) / (16 * nt));
         const long c = (tiles + cus - 1) / cus * (nt + 1);
@@ -403,8 +419,7 @@ static hipError_t xg_launch(const uint8_t *w, const float *x, uint8_t *scratch, 
     }
     switch (best) {
     case 2: return xg_go<F, 2>(w, xh, us, y, sh, s);
-    case 3: return xg_go<F, 3>(w, xh, us, y, sh, s);
-    default: return xg_go<F, 4>(w, xh, us, y, sh, s);
+    default: return xg_go<F, 3>(w, xh, us, y, sh, s);
     }
 }
 
