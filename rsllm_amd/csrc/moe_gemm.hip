@@ -21,9 +21,9 @@
 // eight times: 4.4 GB from memory for 1.1 GB of weights.)
 //
 // DS-V4 experts (256 x IQ2_XXS gate/up 2048 x 4096, Q2_K down 4096 x 2048,
-// top-6) at 512 tokens: the call 1062 us, against 1480 us on mf_rows (1143 us
-// before the IQ2_XXS steps were staggered and the loop freed of spilled
-// addresses). Gate/up is bound by the vector work of the decode (about 97
+// top-6) at 512 tokens: gate/up 688 us, down 358 us, the call 1062 us, against
+// 941, 482 and 1480 us on mf_rows (gate/up 803 us before its steps were
+// staggered and the loop freed of spilled addresses). Gate/up is bound by the vector work of the decode (about 97
 // instructions per 16 x 128 weights) and its table reads.
 #include "mfma_formats.h"
 #include "buffer_lds.h"
