@@ -35,7 +35,9 @@ def test_weight_f32_f32_arm(oracle, hip, n_tok, in_dim, out_dim):
     (1, 4096, 256),   # 16 wavefronts a row
     (6, 4096, 256),   # the same, two passes of tokens
     (1, 700, 257),    # two rows in one workgroup, three tiles, a ragged one
-    (5, 1030, 600),   # three rows a workgroup, splits of unequal length
+    (1, 1030, 600),   # three rows a workgroup, splits of unequal length
+    (5, 1030, 600),   # several tokens: unsplit
+    (3, 2050, 200),   # eight wavefronts a row, nine tiles, three tokens
     (2, 513, 1),      # one row
 ])
 def test_weight_f32_split_rows(oracle, hip, n_tok, in_dim, out_dim):
