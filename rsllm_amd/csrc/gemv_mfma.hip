@@ -850,8 +850,11 @@ __device__ __forceinline__ void mf_x_column(V val4, int in_dim, int t, _Float16 
         hilo8(a, b, up, hi, lo);
         store(i, hi, lo);
         if (sums) {  // two neighbouring threads hold a sub-block of 16
-            float s = ((a.x + a.y) + (a.z + a.w)) + ((b.x + b.y) + (b.z + b.w));
-            s = (s + __shfl_xor(s, 1, 64)) * (up * 0.0625f);
+            // (scaled before they are added, as the image's values: 16 of the
+            // row's largest may pass f32's range, 2^15 each never does)
+            float s = ((a.x * up + a.y * up) + (a.z * up + a.w * up)) +
+                      ((b.x * up + b.y * up) + (b.z * up + b.w * up));
+            s = (s + __shfl_xor(s, 1, 64)) * 0.0625f;
             if ((i & 1) == 0) {
                 const _Float16 h = (_Float16)s;
                 _Float16 *p = sums + (i >> 5) * 32 + ((i >> 1) & 15);

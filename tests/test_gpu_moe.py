@@ -281,6 +281,32 @@ def test_moe_16_slot_dsv4_formats(oracle, hip, n_embd, n_ff, n_tok, k):
         assert np.abs(g - e).max() <= MFMA_TOL * max(np.abs(e).max(), 1e-30)
 
 
+@pytest.mark.parametrize("dt_d", [G.Q2_K, G.IQ2_XXS])
+def test_moe_16_slot_q2k_sums_of_huge_activations(oracle, hip, dt_d):
+    """Q2_K gate/up through the sub-block sums, with activations whose sums
+    over 16 elements pass f32's range while every product of the reference
+    stays inside it: finite, and equal to the oracle (gate and up are far past
+    the clamp, so the output is no less exact than for ordinary tokens)."""
+    n_tok, n_embd, n_ff = 368, 2048, 2048
+    gate, up, down, x, ids, w = make_case(n_tok, n_embd, n_ff, 1, 1, G.Q2_K, dt_d, 700)
+    x[3] = 0.0
+    x[3, 48:64] = 3e37                  # one sub-block: its sum is 4.8e38
+    x[5] = 0.0
+    x[5, 0:2048:128] = 1e37
+    x[5, 1024:1040] = -2.5e37           # -4e38, in another block
+    got = np.zeros(n_tok * n_embd, np.float32)
+    hip.moe_routed(got, x.reshape(-1), gate, up, down, ids, w, n_tok, n_embd, n_ff, 1, 1, G.Q2_K,
+                   dt_d, 10.0)
+    toks = np.array([2, 3, 4, 5])
+    want = run_oracle(oracle, np.zeros(len(toks) * n_embd, np.float32), x[toks], gate, up, down,
+                      ids[toks], w[toks], len(toks), n_embd, n_ff, 1, 1, G.Q2_K, dt_d)
+    assert np.isfinite(want).all()
+    for t, e in zip(toks, want.reshape(len(toks), n_embd)):
+        g = got.reshape(n_tok, n_embd)[t]
+        assert np.isfinite(g).all(), t
+        assert np.abs(g - e).max() <= MFMA_TOL * np.abs(e).max(), t
+
+
 def test_moe_grouped_q6k_full_range_scales(oracle, hip):
     """Q6_K experts whose scales span the whole int8 range (sc (q - 32) up to
     4096, past f16's exact integers) on the grouped matrix-core route: the
