@@ -1564,12 +1564,13 @@ template <class F>
 static hipError_t mfg_gemv(const uint8_t *w0, const uint8_t *w1, size_t w_stride,
                            const _Float16 *xh, const _Float16 *sums, const float *us, int n_rows,
                            const int *tok, const MfgBatch *bat, const int *n_bat, int max_b,
-                           float *y0, float *y1, int in_dim, int out_dim, int bw, hipStream_t s) {
+                           float *y0, float *y1, int in_dim, int out_dim, int bw, bool xm,
+                           hipStream_t s) {
     const uint32_t plane = (uint32_t)((size_t)n_rows * in_dim * 2);
-    // the DS-V4 expert formats, 16-slot batches: weights and activations
-    // staged through LDS
+    // the DS-V4 expert formats, 16-slot batches that fill the chip (xm): weights
+    // and activations staged through LDS
     if constexpr (std::is_same<F, MIQ2>::value || std::is_same<F, MQ2K>::value) {
-        if (bw == kMfgBatch) {
+        if (xm) {
             const uint32_t dt = std::is_same<F, MIQ2>::value ? T_IQ2_XXS : T_Q2_K;
             const hipError_t e = launch_moe_gemm16(dt, w0, w1, w_stride, xh, (size_t)n_rows * in_dim * 4,
                                                    sums, sums ? (size_t)n_rows * (in_dim / 4) : 0, us,
@@ -1651,9 +1652,9 @@ static hipError_t mfg_gemv_dt(uint32_t dt, const uint8_t *w0, const uint8_t *w1,
                               const _Float16 *xh, const _Float16 *sums, const float *us,
                               int n_rows, const int *tok, const MfgBatch *bat, const int *n_bat,
                               int max_b, float *y0, float *y1, int in_dim, int out_dim, int bw,
-                              hipStream_t s) {
+                              bool xm, hipStream_t s) {
     MFG_DT(dt, mfg_gemv<F>(w0, w1, w_stride, xh, sums, us, n_rows, tok, bat, n_bat, max_b, y0, y1,
-                           in_dim, out_dim, bw, s))
+                           in_dim, out_dim, bw, xm, s))
 }
 
 static hipError_t mfg_swiglu_image_dt(uint32_t dt, const float *hg, const float *hu,
@@ -1701,22 +1702,24 @@ hipError_t launch_moe_mfma(uint32_t dt_gu, uint32_t dt_d, const uint8_t *gate, c
     _Float16 *xh2 = reinterpret_cast<_Float16 *>(take((size_t)n_pairs * n_ff * 4));
     _Float16 *sm2 = reinterpret_cast<_Float16 *>(take((size_t)n_pairs * n_ff / 4));
     float *us2 = reinterpret_cast<float *>(take((size_t)n_pairs * 4));
-    if (bw != kMfgBatch || !moe_gemm_sums(dt_gu)) sm1 = nullptr;
-    if (bw != kMfgBatch || !moe_gemm_sums(dt_d)) sm2 = nullptr;
+    const bool xm1 = bw == kMfgBatch && moe_gemm16_fills(dt_gu, n_embd, n_ff, 2, n_pairs, n_expert);
+    const bool xm2 = bw == kMfgBatch && moe_gemm16_fills(dt_d, n_ff, n_embd, 1, n_pairs, n_expert);
+    if (!xm1 || !moe_gemm_sums(dt_gu)) sm1 = nullptr;
+    if (!xm2 || !moe_gemm_sums(dt_d)) sm2 = nullptr;
     hipError_t e;
     // routing (when given) and the x image in one launch
     if ((e = mfg_route_x_dt(dt_gu, route, bat, n_bat, bw, x, n_tok, xh1, us1, n_embd, sm1, s)) !=
         hipSuccess)
         return e;
     if ((e = mfg_gemv_dt(dt_gu, gate, up, gu_stride, xh1, sm1, us1, n_tok, slot_tok, bat, n_bat, max_b,
-                         hg, hu, n_embd, n_ff, bw, s)) != hipSuccess)
+                         hg, hu, n_embd, n_ff, bw, xm1, s)) != hipSuccess)
         return e;
     // off[n_expert]: the routed slot count
     if ((e = mfg_swiglu_image_dt(dt_d, hg, hu, off + n_expert, n_pairs, clamp, xh2, us2, n_ff,
                                  sm2, s)) != hipSuccess)
         return e;
     return mfg_gemv_dt(dt_d, down, nullptr, d_stride, xh2, sm2, us2, n_pairs, nullptr, bat, n_bat,
-                       max_b, yd, nullptr, n_ff, n_embd, bw, s);
+                       max_b, yd, nullptr, n_ff, n_embd, bw, xm2, s);
 }
 
 bool lora_mfma_supported(uint32_t dtype, int n_tok, int D, int G, int R) {

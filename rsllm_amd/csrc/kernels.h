@@ -181,6 +181,10 @@ hipError_t launch_moe_mfma(uint32_t dt_gu, uint32_t dt_d, const uint8_t *gate, c
 // scaled row's sums over 16 elements as 16 hi then 16 lo planes.
 // hipErrorNotSupported for formats, alignments or in_dim it does not take.
 inline bool moe_gemm_sums(uint32_t dtype) { return dtype == T_Q2_K; }
+// Whether a call of n_pairs slots over n_expert experts fills this kernel's
+// workgroups (mats matrices of out_dim rows an expert); callers keep k_gemv_mfg
+// where it does not.
+bool moe_gemm16_fills(uint32_t dtype, int in_dim, int out_dim, int mats, int n_pairs, int n_expert);
 hipError_t launch_moe_gemm16(uint32_t dtype, const uint8_t *w0, const uint8_t *w1, size_t w_stride,
                              const void *xh, size_t x_bytes, const void *sums, size_t s_bytes,
                              const float *us, const int *tok, const MfgBatch *bat, const int *n_bat, int max_b, float *y0, float *y1,

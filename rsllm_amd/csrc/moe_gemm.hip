@@ -25,6 +25,9 @@
 // 941, 482 and 1480 us on mf_rows (gate/up 803 us before its steps were
 // staggered and the loop freed of spilled addresses). Gate/up is bound by the vector work of the decode (about 97
 // instructions per 16 x 128 weights) and its table reads.
+#include <algorithm>
+#include <cmath>
+
 #include "mfma_formats.h"
 #include "buffer_lds.h"
 
@@ -414,6 +417,30 @@ static hipError_t xm_go(const uint8_t *w0, const uint8_t *w1, size_t w_stride, c
     k_xm<F><<<g, 64 * kXmNW, LDS, s>>>(w0, w1, w_stride, xh, x_bytes, sums, s_bytes, us, tok, bat,
                                        n_bat, y0, y1, in_dim, out_dim);
     return hipGetLastError();
+}
+
+// One workgroup fits a CU and takes the same time whether or not the others are
+// busy, so this kernel pays once most CUs of every round have one: against
+// k_gemv_mfg, by workgroups per round of 256 CUs (kernel times, us; IQ2_XXS
+// gate/up of K 4096: 16: 20 -> 60, 64: 44 -> 65, 96: 52 -> 66, 128: 65 -> 68,
+// 144: 74 -> 68, 192: 85 -> 73, 234: 98 -> 73; two rounds of 144: 126 -> 140, of
+// 192: 169 -> 145, of 256: 209 -> 158; Q2_K down of K 2048: 64: 22 -> 32, 128: 32
+// -> 33, 144: 38 -> 34, 192: 45 -> 35; K 8192 the same by the round). The line
+// is where all of the traced shapes win or are level: seven tenths of the CUs
+// for IQ2_XXS, whose workgroups also stage the tables (three rounds of 172, 64
+// experts of 2048 x 2048 at 9 slots: the call 191 -> 207; of 184: 233 -> 197 for
+// the gate/up of 8 experts at 130), six tenths for Q2_K. The number of batches
+// is known on the device alone; this is what slots dealt evenly at random make:
+// with m a mean expert's slots, m / 16 batches and half of one more each, and
+// below 18 slots, where few experts have a second batch, about 1 + (m - 8)^2 /
+// 150.
+bool moe_gemm16_fills(uint32_t dtype, int in_dim, int out_dim, int mats, int n_pairs, int n_expert) {
+    if ((dtype != T_IQ2_XXS && dtype != T_Q2_K) || in_dim % 2048 != 0) return false;
+    const double m = (double)n_pairs / n_expert;
+    const double batches = n_expert * std::min(m / 16 + 0.5, 1 + (m - 8) * (m - 8) / 150);
+    const double wgs = batches * ((out_dim + kXmRows - 1) / kXmRows) * mats;
+    const double cus = device_cus();
+    return wgs >= (dtype == T_IQ2_XXS ? 0.7 : 0.6) * cus * std::ceil(wgs / cus);
 }
 
 hipError_t launch_moe_gemm16(uint32_t dtype, const uint8_t *w0, const uint8_t *w1, size_t w_stride,

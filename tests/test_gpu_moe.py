@@ -281,6 +281,72 @@ def test_moe_16_slot_dsv4_formats(oracle, hip, n_embd, n_ff, n_tok, k):
         assert np.abs(g - e).max() <= MFMA_TOL * max(np.abs(e).max(), 1e-30)
 
 
+def _call_us(hip, dt_gu, dt_d, n_tok, n_expert, n_embd, n_ff):
+    """GPU time of one routed-expert call, the smallest of several in a row."""
+    import torch
+    gate, up, down, x, ids, w = make_case(n_tok, n_embd, n_ff, n_expert, 1, dt_gu, dt_d, 40)
+    ids[:, 0] = np.arange(n_tok) % n_expert
+    s = torch.cuda.current_stream().cuda_stream
+    dev = []
+    for raw, dt, ind in ((gate, dt_gu, n_embd), (up, dt_gu, n_embd), (down, dt_d, n_ff)):
+        r = torch.from_numpy(raw).cuda()
+        d = torch.empty_like(r)
+        hip.prepare_weights_dev(d.data_ptr(), r.data_ptr(), r.numel(), dt, ind, s)
+        dev.append(d)
+    dx, di, dw = (torch.from_numpy(a.reshape(-1)).cuda() for a in (x, ids, w))
+    y = torch.zeros(n_tok * n_embd, device="cuda")
+    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    best = float("inf")
+    for i in range(40):
+        a.record()
+        for _ in range(10):
+            hip.moe_routed_dev(y.data_ptr(), y.numel(), dx.data_ptr(), dx.numel(), dev[0].data_ptr(),
+                               dev[1].data_ptr(), dev[0].numel(), dev[2].data_ptr(),
+                               dev[2].numel(), di.data_ptr(), dw.data_ptr(), n_tok, n_tok, n_embd,
+                               n_ff, n_expert, 1, dt_gu, dt_d, 10.0, s)
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) * 100.0)
+    return best
+
+
+@pytest.mark.parametrize("dt_gu,dt_d", [(G.IQ2_XXS, G.Q2_K), (G.Q2_K, G.IQ2_XXS)])
+@pytest.mark.parametrize("n_expert", [4, 8])
+def test_moe_16_slot_batches_of_few_experts_are_not_slow(hip, dt_gu, dt_d, n_expert):
+    """The first token past 8 slots an expert moves a call to 16-slot batches.
+    With a few experts the 512-row workgroups of the staged kernel would leave
+    most CUs idle (2.4 to 3.5 times the call at 8 slots measured); the 64-row
+    ones of the unstaged kernel measured 1.36 to 1.73 times."""
+    at8 = _call_us(hip, dt_gu, dt_d, 8 * n_expert, n_expert, 4096, 2048)
+    past = _call_us(hip, dt_gu, dt_d, 8 * n_expert + 1, n_expert, 4096, 2048)
+    print(f"{dt_gu.name}/{dt_d.name} {n_expert} experts: {at8:.1f} us at 8 slots, {past:.1f} past")
+    assert past <= 2.1 * at8
+
+
+@pytest.mark.parametrize("dt_gu,dt_d,n_embd,n_ff,n_tok", [
+    (G.IQ2_XXS, G.Q2_K, 4096, 2048, 193),   # 12 full batches an expert and one of one slot
+    (G.Q2_K, G.IQ2_XXS, 4096, 2048, 193),   # sums of two matrices' x found through the tokens
+    (G.Q2_K, G.Q2_K, 2048, 4096, 369),      # sums on both sides, down over two super-tiles
+    (G.IQ2_XXS, G.IQ2_XXS, 2304, 2048, 305),  # rows in a partial block; gate and up unstaged
+    (G.Q2_K, G.Q2_K, 2048, 2304, 161),      # gate and up in a partial block; down unstaged
+])
+def test_moe_16_slot_staged_pairings(oracle, hip, dt_gu, dt_d, n_embd, n_ff, n_tok):
+    """Enough batches for the staged 16-slot kernel, every token on both
+    experts: each pairing of its formats, of its rows and of its K."""
+    gate, up, down, x, ids, w = make_case(n_tok, n_embd, n_ff, 2, 2, dt_gu, dt_d, 860 + n_tok)
+    x[1] = np.abs(x[1])  # large sub-block sums
+    w[2, 0] = 0.0        # a skipped slot
+    got = np.zeros(n_tok * n_embd, np.float32)
+    hip.moe_routed(got, x.reshape(-1), gate, up, down, ids, w, n_tok, n_embd, n_ff, 2, 2, dt_gu,
+                   dt_d, 10.0)
+    toks = np.array([0, 1, 2, 15, 16, n_tok - 1])
+    want = run_oracle(oracle, np.zeros(len(toks) * n_embd, np.float32), x[toks], gate, up, down,
+                      ids[toks], w[toks], len(toks), n_embd, n_ff, 2, 2, dt_gu, dt_d)
+    got, want = got.reshape(n_tok, n_embd)[toks], want.reshape(len(toks), n_embd)
+    for g, e in zip(got, want):
+        assert np.abs(g - e).max() <= MFMA_TOL * np.abs(e).max()
+
+
 @pytest.mark.parametrize("dt_d", [G.Q2_K, G.IQ2_XXS])
 def test_moe_16_slot_q2k_sums_of_huge_activations(oracle, hip, dt_d):
     """Q2_K gate/up through the sub-block sums, with activations whose sums
