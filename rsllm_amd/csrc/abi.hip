@@ -590,16 +590,30 @@ int lora_down_compute(float *out, size_t out_len, const uint8_t *w, size_t strid
         return ok();
     }
     hipError_t e = hipErrorNotSupported;
-    // Prompts: the many-token GEMM, once the 16-token passes below would make
-    // more than about five workgroups per two CUs, or from 256 tokens (which
-    // pay for its longer workgroups on few rows): passes against GEMM, 8 x
-    // [1024 x 4096] Q8_0 52 vs 54 us at 64 tokens, 74 vs 56 at 96, 236 vs 83
-    // at 300; 4 x [512 x 2048] 23 vs 32 at 96, 47 vs 35 at 300; 16 x [256 x
-    // 1024] 20 vs 23 at 96, 27 vs 25 at 160; 8 x [128 x 4096] 44 vs 54 at
-    // 160, 78 vs 59 at 300.
-    const long passes_wg = ((long)T + 15) / 16 * ((long)G * R / 64);
-    if (!group_layout && (passes_wg >= 640 || T >= 256) && T > 32 &&
-        gemm_exact_supported(dtype, T, D, G, R)) {
+    // Prompts: the many-token GEMM, once the 16-token passes below make more
+    // than about five workgroups per two CUs or the prompt has 256 tokens, and
+    // they make that many without their images of 16 tokens of a group, each
+    // of which weighs as much as ten workgroups: with few groups and rows the
+    // GEMM's 256-row tiles leave most CUs idle. Rows of whole 2048 elements
+    // need the first alone (the passes read the tokens of such images from few
+    // L2 channels). Passes against GEMM, us:
+    //   8 x [1024 x 4096] Q8_0 52 / 54 at 64 tokens, 74 / 56 at 96, 236 / 83 at
+    //   300; 4 x [512 x 2048] 23 / 32 at 96, 47 / 35 at 300; 16 x [256 x 1024]
+    //   20 / 23 at 96, 27 / 25 at 160; 8 x [128 x 4096] 44 / 54 at 160, 55 / 56
+    //   at 256, 84 / 60 at 352; 4 x [256 x 4096] 41 / 58 at 256, 65 / 58 at 352;
+    //   2 x [512 x 4096] 33 / 54 at 256, 61 / 57 at 512; 1 x [1024 x 4096] 32 /
+    //   52 at 256, 52 / 54 at 512, 73 / 55 at 640; 1 x [1024 x 256] 9 / 10 at
+    //   512, 13 / 11 at 640; 1 x [8192 x D] at 80 (640 workgroups, 5 images)
+    //   16 / 18 at D = 1024, 38 / 41 at 3072, but 36 / 30 at 2048, 66 / 52 at
+    //   4096.
+    // Shapes those passes refuse run 8 tokens a launch otherwise (4 x [192 x
+    // 1024] 163 / 20 at 300); they start at the same number of tokens, which
+    // was not measured for them.
+    const long chunks = ((long)T + 15) / 16 * G, passes_wg = chunks * R / 64;
+    const bool many = (passes_wg >= 640 || T >= 256) &&
+                      (passes_wg + 10 * chunks >= 1024 || (passes_wg >= 640 && D % 2048 == 0) ||
+                       !lora_mfma_supported(dtype, T, D, G, R));
+    if (!group_layout && many && T > 32 && gemm_exact_supported(dtype, T, D, G, R)) {
         HIP_TRY(sc.xq.ensure(gemm_exact_scratch_bytes(T, D, G)), "hipMalloc");
         e = launch_gemm_exact(dtype, w, stride * n_groups, x, (uint8_t *)sc.xq.p, out, T, D, G, R,
                               tout, s);

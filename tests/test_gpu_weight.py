@@ -300,3 +300,32 @@ def test_grouped_lora_down_many_token_gemm(oracle, hip, n_groups, group_dim, ran
     assert not np.isnan(got).any()
     for k, t in enumerate(toks):
         assert rel_err(got.reshape(n_tok, -1)[t], want[k]) <= 2e-5
+
+
+@pytest.mark.parametrize("n_groups,rank", [(1, 1024), (2, 512), (4, 256)])
+def test_grouped_lora_down_256_tokens_of_few_groups_are_not_slow(hip, n_groups, rank):
+    """Few groups and ranks leave most CUs without a 256-row tile of the
+    many-token GEMM; the 16-token passes keep the 256th token as cheap as the
+    255th (with the GEMM it cost 1.4 to 1.7 times the call)."""
+    import torch
+    group_dim = 4096
+    w, x = grouped_case(G.Q8_0, 256, n_groups, group_dim, rank, 40)
+    s = torch.cuda.current_stream().cuda_stream
+    d_raw, d_x = torch.from_numpy(w.copy()).cuda(), torch.from_numpy(x.reshape(-1).copy()).cuda()
+    d_w = torch.empty_like(d_raw)
+    hip.prepare_weights_dev(d_w.data_ptr(), d_raw.data_ptr(), w.size, G.Q8_0, group_dim, s)
+    d_y = torch.empty(256 * n_groups * rank, device="cuda")
+    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    us = {255: float("inf"), 256: float("inf")}
+    for i in range(80):
+        t = 255 + i % 2
+        a.record()
+        for _ in range(10):
+            hip.matmul_grouped_lora_down_dev(d_y.data_ptr(), t * n_groups * rank, d_w.data_ptr(),
+                                             d_w.numel(), d_x.data_ptr(), t * n_groups * group_dim,
+                                             t, n_groups, group_dim, rank, G.Q8_0, s)
+        b.record()
+        b.synchronize()
+        us[t] = min(us[t], a.elapsed_time(b) * 100.0)
+    print(f"{n_groups} x [{rank} x {group_dim}]: {us[255]:.1f} us at 255 tokens, {us[256]:.1f} at 256")
+    assert us[256] <= 1.25 * us[255]
