@@ -102,6 +102,20 @@ struct DevBuf {
     }
 };
 
+// Whether `b` holds n bytes, grown where that takes it. False, with no error
+// left behind, where it cannot grow: no memory, or `s` is being captured (an
+// allocation would end the capture). For routes that have another to give way
+// to.
+bool workspace(DevBuf &b, size_t n, hipStream_t s) {
+    if (n <= b.cap) return true;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone &&
+        b.ensure(n) == hipSuccess)
+        return true;
+    (void)hipGetLastError();
+    return false;
+}
+
 // Pinned host staging for the activations and outputs of the host-pointer
 // entry points. A small copy from or to pageable memory costs the runtime a
 // blocking round trip (4096 x 4096 Q4_K, one token, 16 KB each way: 33.8 us a
@@ -613,12 +627,13 @@ int lora_down_compute(float *out, size_t out_len, const uint8_t *w, size_t strid
     const bool many = (passes_wg >= 640 || T >= 256) &&
                       (passes_wg + 10 * chunks >= 1024 || (passes_wg >= 640 && D % 2048 == 0) ||
                        !lora_mfma_supported(dtype, T, D, G, R));
-    if (!group_layout && many && T > 32 && gemm_exact_supported(dtype, T, D, G, R)) {
-        HIP_TRY(sc.xq.ensure(gemm_exact_scratch_bytes(T, D, G)), "hipMalloc");
+    // (the routes after it need less workspace, the last of them none)
+    if (!group_layout && many && T > 32 &&
+        gemm_exact_supported(dtype, w, stride * n_groups, x, T, D, G, R) &&
+        workspace(sc.xq, gemm_exact_scratch_bytes(T, D, G), s)) {
         e = launch_gemm_exact(dtype, w, stride * n_groups, x, (uint8_t *)sc.xq.p, out, T, D, G, R,
                               tout, s);
-        if (e == hipSuccess) return ok();
-        if (e != hipErrorNotSupported) return dev_err(e, "gemm_exact");
+        return e == hipSuccess ? ok() : dev_err(e, "gemm_exact");
     }
     // 9 or more tokens of the matrix-core formats: one pass over the stacked
     // matrix per 16 tokens, on the matrix cores

@@ -428,16 +428,17 @@ size_t gemm_exact_scratch_bytes(int n_tok, int in_dim, int groups) {
     return rows * xg_row_bytes(in_dim) + rows * 4;
 }
 
-bool gemm_exact_supported(uint32_t dtype, int n_tok, int in_dim, int groups, int group_rows) {
+bool gemm_exact_supported(uint32_t dtype, const uint8_t *w, size_t w_bytes, const float *x,
+                          int n_tok, int in_dim, int groups, int group_rows) {
     return dtype == T_Q8_0 && n_tok > 0 && in_dim > 0 && in_dim % 256 == 0 && group_rows > 0 &&
-           (size_t)n_tok * groups * xg_row_bytes(in_dim) <= 0x7FFFFFFFu;
+           (size_t)n_tok * groups * xg_row_bytes(in_dim) <= 0x7FFFFFFFu && w_bytes <= 0xFFFFFF00u &&
+           (((uintptr_t)w | (uintptr_t)x) & 15) == 0;
 }
 
 hipError_t launch_gemm_exact(uint32_t dtype, const uint8_t *w, size_t w_bytes, const float *x,
                              uint8_t *scratch, float *y, int n_tok, int in_dim, int groups,
                              int group_rows, int y_stride, hipStream_t s) {
-    if (!gemm_exact_supported(dtype, n_tok, in_dim, groups, group_rows) || w_bytes > 0xFFFFFF00u ||
-        (((uintptr_t)w | (uintptr_t)x) & 15) != 0)
+    if (!gemm_exact_supported(dtype, w, w_bytes, x, n_tok, in_dim, groups, group_rows))
         return hipErrorNotSupported;
     const XgShape sh{in_dim, n_tok, groups, group_rows, y_stride,
                      (uint32_t)((size_t)n_tok * groups * xg_row_bytes(in_dim)), (uint32_t)w_bytes};

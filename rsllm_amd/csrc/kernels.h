@@ -207,9 +207,11 @@ hipError_t launch_lora_mfma(uint32_t dtype, const uint8_t *w, size_t w_bytes, co
 // group_rows + r, i] x[(t * groups + g) * in_dim + i] for a matrix of groups *
 // group_rows rows (device layout as one matrix), the weights exact and the
 // activations as hi + lo f16. `scratch` holds gemm_exact_scratch_bytes bytes.
-// Q8_0; hipErrorNotSupported outside gemm_exact_supported or where w or x is
-// not 16-byte aligned.
-bool gemm_exact_supported(uint32_t dtype, int n_tok, int in_dim, int groups, int group_rows);
+// gemm_exact_supported: Q8_0, whole 256-element blocks, w and x 16-byte
+// aligned, the image and w within 32-bit offsets; launch_gemm_exact refuses
+// the rest with hipErrorNotSupported.
+bool gemm_exact_supported(uint32_t dtype, const uint8_t *w, size_t w_bytes, const float *x,
+                          int n_tok, int in_dim, int groups, int group_rows);
 size_t gemm_exact_scratch_bytes(int n_tok, int in_dim, int groups);
 hipError_t launch_gemm_exact(uint32_t dtype, const uint8_t *w, size_t w_bytes, const float *x,
                              uint8_t *scratch, float *y, int n_tok, int in_dim, int groups,

@@ -329,3 +329,69 @@ def test_grouped_lora_down_256_tokens_of_few_groups_are_not_slow(hip, n_groups, 
         us[t] = min(us[t], a.elapsed_time(b) * 100.0)
     print(f"{n_groups} x [{rank} x {group_dim}]: {us[255]:.1f} us at 255 tokens, {us[256]:.1f} at 256")
     assert us[256] <= 1.25 * us[255]
+
+
+def _lora_dev(hip, w, x, n_groups, group_dim, rank, offset=0):
+    """Device copies of a grouped case (x `offset` floats into its buffer) and
+    a call on a stream; y is returned by the call."""
+    import torch
+    n_tok = len(x)
+    s0 = torch.cuda.current_stream().cuda_stream
+    d_raw = torch.from_numpy(w.copy()).cuda()
+    d_w = torch.empty_like(d_raw)
+    hip.prepare_weights_dev(d_w.data_ptr(), d_raw.data_ptr(), w.size, G.Q8_0, group_dim, s0)
+    buf = torch.zeros(x.size + offset, device="cuda")
+    buf[offset:] = torch.from_numpy(x.reshape(-1).copy()).cuda()
+    d_x, d_y = buf[offset:], torch.full((n_tok, n_groups * rank), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+
+    def call(stream):
+        hip.matmul_grouped_lora_down_dev(d_y.data_ptr(), d_y.numel(), d_w.data_ptr(), w.size,
+                                         d_x.data_ptr(), d_x.numel(), n_tok, n_groups, group_dim,
+                                         rank, G.Q8_0, stream)
+        return d_y
+    return call, d_x
+
+
+def test_grouped_lora_down_prompt_captured_on_a_new_stream(oracle, hip):
+    """A prompt whose rank the 16-token passes refuse, captured on a stream
+    without workspace: the many-token GEMM, which needs some, gives way to the
+    launches that need none. Replays follow the contents of x."""
+    import torch
+    n_tok, n_groups, group_dim, rank = 256, 2, 512, 96
+    w, x = grouped_case(G.Q8_0, n_tok, n_groups, group_dim, rank, 60)
+    toks = np.array([0, 7, 8, 100, 255])
+    want = oracle_grouped(oracle, w, x, toks, n_groups, group_dim, rank, G.Q8_0)
+    call, d_x = _lora_dev(hip, w, x, n_groups, group_dim, rank)
+    call(torch.cuda.current_stream().cuda_stream)  # the library is up before the capture
+    torch.cuda.synchronize()
+    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        d_y = call(s.cuda_stream)
+    for k in range(4):
+        d_y.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert rel_err(d_y.cpu().numpy()[toks], want * 2.0 ** k) <= REL_TOL
+        d_x.mul_(2.0)
+        torch.cuda.synchronize()
+    hip.stream_release(s.cuda_stream)
+
+
+def test_grouped_lora_down_prompt_unaligned_x_needs_no_workspace(oracle, hip):
+    """x 4 bytes past a 16-byte boundary is not for the many-token GEMM: the
+    call takes the launches without workspace and allocates none."""
+    import torch
+    n_tok, n_groups, group_dim, rank = 256, 2, 512, 96
+    w, x = grouped_case(G.Q8_0, n_tok, n_groups, group_dim, rank, 61)
+    toks = np.array([0, 7, 8, 100, 255])
+    want = oracle_grouped(oracle, w, x, toks, n_groups, group_dim, rank, G.Q8_0)
+    call, _ = _lora_dev(hip, w, x, n_groups, group_dim, rank, offset=1)
+    hip.init(0)
+    s = torch.cuda.Stream()
+    before = hip.device_allocations()
+    d_y = call(s.cuda_stream)
+    s.synchronize()
+    assert hip.device_allocations() == before
+    assert rel_err(d_y.cpu().numpy()[toks], want) <= REL_TOL
+    hip.stream_release(s.cuda_stream)
