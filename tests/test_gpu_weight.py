@@ -302,6 +302,31 @@ def test_grouped_lora_down_many_token_gemm(oracle, hip, n_groups, group_dim, ran
         assert rel_err(got.reshape(n_tok, -1)[t], want[k]) <= 2e-5
 
 
+@pytest.mark.parametrize("n_groups,group_dim,rank,n_tok", [
+    # three column tiles a workgroup (more than 256 tiles of two, at most 256
+    # of three)
+    (8, 512, 1024, 300),    # whole row blocks, six whole token tiles and 12 tokens
+    (9, 256, 900, 288),     # 132 rows in the last block (not whole 16s), whole token tiles
+    (8, 768, 1024, 290),    # K of three tiles, 2 tokens in the last token tile
+    # two
+    (3, 512, 384, 400),     # one and a half row blocks, 16 tokens in the last token tile
+    (2, 8448, 40, 256),     # activation rows too long for registers: read twice
+])
+def test_grouped_lora_down_many_token_gemm_tiles(oracle, hip, n_groups, group_dim, rank, n_tok):
+    """Both widths of the many-token GEMM's workgroup, tokens on both sides of
+    their tiles' edges; the bound of test_grouped_lora_down_many_token_gemm."""
+    w, x = grouped_case(G.Q8_0, n_tok, n_groups, group_dim, rank, 930 + n_tok)
+    x[48] *= 1e4  # a token of another scale, the first of a tile of 48
+    toks = np.unique(np.minimum([0, 15, 16, 31, 32, 47, 48, 95, 96, 143, 144, 287, 288, n_tok - 1],
+                                n_tok - 1))
+    want = oracle_grouped(oracle, w, x, toks, n_groups, group_dim, rank, G.Q8_0)
+    got = np.full(n_tok * n_groups * rank, np.nan, np.float32)
+    hip.matmul_grouped_lora_down(got, w, x.reshape(-1), n_tok, n_groups, group_dim, rank, G.Q8_0)
+    assert not np.isnan(got).any()
+    for k, t in enumerate(toks):
+        assert rel_err(got.reshape(n_tok, -1)[t], want[k]) <= 2e-5
+
+
 @pytest.mark.parametrize("n_groups,rank", [(1, 1024), (2, 512), (4, 256)])
 def test_grouped_lora_down_256_tokens_of_few_groups_are_not_slow(hip, n_groups, rank):
     """Few groups and ranks leave most CUs without a 256-row tile of the
