@@ -12,21 +12,26 @@
 //    steps of 64 elements. Wavefront w holds two row tiles (rows 32 (w & 7)
 //    ..) for all columns and 32 elements of each step (K group w >> 3): four
 //    wavefronts per SIMD, since one alone issues vector work at about half
-//    rate and the decode and the block scales need as much as the MFMAs. Weights (raw bytes) and activations reach LDS by 16-byte
-//    buffer-to-LDS pieces: the activations through a ring of four steps, the
+//    rate and the decode and the block scales need as much as the MFMAs.
+//    Weights (raw bytes) and activations reach LDS by 16-byte buffer-to-LDS
+//    pieces: the activations through a ring of four steps, the
 //    weights one 256-element tile at a time (a row's tile is one contiguous
 //    run: few cache lines per instruction), which every wavefront reads into
 //    registers a step before it needs it, so the buffer takes the next tile
 //    while this one is computed. A step's operands are decoded during the
 //    step before. The K groups' sums are added through LDS at the end.
 //
-// 8 x [1024 x 4096] Q8_0 at 300 tokens: 74 us (40 GFLOP counting both planes,
-// 0.54 PFLOP/s) after 16 us for the image (79 MB at 4.9 TB/s), against 197 +
-// 38 us for the 16-token passes. What bounds it: per 32 x 16 x 16 products
-// two MFMAs (32 cycles), 4 FMAs for the block scales and a share of the
-// decode, with the copies and the LDS reads of the activations beside them.
+// 8 x [1024 x 4096] Q8_0 at 300 tokens, kernel trace over three sets of
+// operands in turn: 78 us (72 at best; 40 GFLOP counting both planes, 0.51
+// PFLOP/s) after 17 us for the image (39 MB read and 79 MB written, part of it
+// in the last-level cache), against 197 + 38 us for the 16-token passes. Calls
+// one after the other overlap at their ends: 82 us each (74 on one set of
+// operands). What bounds it: per 32 x 16 x 16 products two MFMAs (32 cycles),
+// 4 FMAs for the block scales and a share of the decode, with the copies and
+// the LDS reads of the activations beside them.
 //
-// (Tried on that shape: the weights straight to the operand registers, each
+// (Tried on that shape, before the tile sums, when the kernel's trace read 74
+// us: the weights straight to the operand registers, each
 // lane its own row, 107 us: neighbouring lanes hit 64 different lines per
 // instruction. Both through two buffers of 128 elements, 76 us; both through
 // a ring of four 64-element steps, 89 us: a row's 64 bytes and its scales per
@@ -392,7 +397,10 @@ static hipError_t xg_go(const uint8_t *w, const _Float16 *xh, const float *us, f
 
 // Column tiles per workgroup: the fewest (rounds of one workgroup per CU) x
 // (work of one), counting one column tile's time for what a workgroup does
-// whatever its width. Four do not fit the registers beside the tile sums (65
+// whatever its width. That picked the faster of the two in all of 159 measured
+// calls (3 to 16 groups, K of 512 to 4096, 256 to 1000 tokens): 8 x [1024 x
+// 4096] at 256 / 300 / 400 / 640 tokens two tiles 63 / 109 / 115 / 174 us, three
+// 69 / 73 / 132 / 148. Four do not fit the registers beside the tile sums (65
 // spilled); with one chain of sums instead they served 16 x [512 x 1024] at
 // 400 tokens in 34 us (three: 42 us, the 16-token passes 76 us) at an error
 // above the passes' own (1.1e-7 against 9.9e-8; now 9.6e-8).

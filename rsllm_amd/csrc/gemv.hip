@@ -879,7 +879,8 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_f32(const float *__restrict__ 
 // wavefronts (wavefront w: row slot w / KS, tiles w % KS, w % KS + KS, ..),
 // whose sums are added through LDS in order. With one row per workgroup
 // k_gemv_f32 runs one wavefront of 16 and waits out its tiles' latency one
-// after the other: the 256 x 4096 router at one token took 11.7 us, here 3.7.
+// after the other: the 256 x 4096 router at one token, in a chain of calls
+// (weights from memory), took 11.7 us, here 3.6.
 template <int NW, int BT>
 __global__ __launch_bounds__(64 * NW) void k_gemv_f32_split(const float *__restrict__ w,
                                                            const float *__restrict__ x,
@@ -946,13 +947,18 @@ hipError_t launch_gemv_f32(const float *w, const float *x, float *y, int n_tok, 
     const size_t per = ((size_t)1 << 29) / (size_t)(x_stride > 0 ? x_stride : 1);
     const int chunk = per == 0 ? 1 : per > (size_t)n_tok ? n_tok : (int)per;
     // wavefronts per row: as many as fill the workgroup, at most a tile of 256
-    // elements each
+    // elements each (one token, kernel times unsplit / split, us: 256 rows of
+    // 512 4.3 / 4.1, of 1024 4.2 / 3.9, of 2048 5.6 / 4.4; 2048 rows of 512 4.1 /
+    // 4.2, of 1024 5.4 / 4.2, of 2048 7.8 / 4.6; calls of K 16384: 256 rows 33 /
+    // 4.9, 2048 rows 42 / 21; level with one or two tiles, never slower by more
+    // than the runs differ)
     const int rows_wg = (out_dim + n_wg - 1) / n_wg, tiles = (in_dim + 255) / 256;
     int ks = 1;
     while (2 * ks * rows_wg <= 16 && 2 * ks <= tiles) ks *= 2;
     // Several tokens only where one row's K keeps eight or more wavefronts
-    // busy (256 x 4096 at 8 / 128 tokens: 15.2 / 290 us unsplit, 5.5 / 62
-    // split): more rows fill the workgroup themselves, and the unsplit kernel
+    // busy (256 x 4096 at 8 / 128 tokens: 15.3 / 214 us unsplit, 5.6 / 52
+    // split; 200 x 2048 8.9 / 114 and 4.8 / 40; 128 x 16384 53 / 1106 and 17 /
+    // 582): more rows fill the workgroup themselves, and the unsplit kernel
     // streams better (1500 x 2048 at 64 tokens: 86 us, 242 split in two).
     if (n_tok > 1 && (rows_wg > 1 || ks < 8)) ks = 1;
     for (int t0 = 0; t0 < n_tok; t0 += chunk) {

@@ -23,8 +23,10 @@
 // DS-V4 experts (256 x IQ2_XXS gate/up 2048 x 4096, Q2_K down 4096 x 2048,
 // top-6) at 512 tokens: gate/up 688 us, down 358 us, the call 1062 us, against
 // 941, 482 and 1480 us on mf_rows (gate/up 803 us before its steps were
-// staggered and the loop freed of spilled addresses). Gate/up is bound by the vector work of the decode (about 97
-// instructions per 16 x 128 weights) and its table reads.
+// staggered and the loop freed of spilled addresses). Gate/up is bound by the
+// vector work of the decode (about 97 instructions per 16 x 128 weights) and
+// its table reads. Calls whose workgroups leave CUs idle stay on mf_rows
+// (moe_gemm16_fills).
 #include <algorithm>
 #include <cmath>
 
@@ -51,8 +53,9 @@ __device__ __forceinline__ void xm_stage_tables(uint4 *tab, int threads) {
 // 4); so: the super-tile's offset, half hf); load_aux(): what serves the whole
 // half, into the next half's fields (rr: row r16's offset), next(): makes it
 // current. put(): block b's bytes into the wavefront's LDS rows (stride 80
-// bytes; row lane / 4, piece lane % 4). Then step() adds the MFMAs of step half
-// h of block b (128 elements) and fold() closes the block.
+// bytes; row lane / 4, piece lane % 4); put_half(): those of the half's scales.
+// Then step() adds the MFMAs of step half h of block b (128 elements) and
+// fold() closes the block, or step_all() does both for all row tiles.
 constexpr int kXmRow = 80;  // LDS bytes per row: 16 rows spread over the banks
 template <class F> struct XmFmt;
 template <> struct XmFmt<MIQ2> {
@@ -72,7 +75,6 @@ template <> struct XmFmt<MIQ2> {
         dn = bload8(r, rr + 512u, so + 8u * (uint32_t)hf);
     }
     __device__ void next() { d = dn; }
-    __device__ void put_half(uint8_t *, int) const {}
     __device__ void put(uint8_t *buf, int lane, int b) const {
         *reinterpret_cast<uint4 *>(buf + (lane >> 2) * kXmRow + 16 * (lane & 3)) = qs[b];
     }
@@ -173,7 +175,7 @@ template <> struct XmFmt<MQ2K> {
         *reinterpret_cast<uint4 *>(buf + (lane >> 2) * kXmRow + 16 * (lane & 3)) = qs[b];
     }
     __device__ void step(const uint8_t *buf, int r16, int q, int b, int h, const uint4 (&x)[4],
-                         const uint4 (&xl)[4], f32x4 &P, f32x4 &, const uint8_t *) const {
+                         const uint4 (&xl)[4], f32x4 &P) const {
         const uint2 v = *reinterpret_cast<const uint2 *>(buf + r16 * kXmRow + 32 * h + 8 * q);
         const uint2 sc = *reinterpret_cast<const uint2 *>(buf + 16 * kXmRow + r16 * kXmRow + 16 * b + 8 * h);
         // scale bytes 2 j + q / 2, j = 0..3, as f16 sc 2^(9 - 2 j)
@@ -345,9 +347,10 @@ __global__ __launch_bounds__(64 * kXmNW) void k_xm(const uint8_t *__restrict__ w
         }
         if constexpr (i == 7) load_w(hb + 1, 1);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (i == 0)
+        if constexpr (G::SN != 0)
+            if constexpr (i == 0)
 #pragma unroll
-            for (int rt = 0; rt < RT; rt++) wc[rt].put_half(wbuf + rt * X::kBuf, lane);
+                for (int rt = 0; rt < RT; rt++) wc[rt].put_half(wbuf + rt * X::kBuf, lane);
         if constexpr (h == 0)
 #pragma unroll
             for (int rt = 0; rt < RT; rt++) wc[rt].put(wbuf + rt * X::kBuf, lane, b);
@@ -372,7 +375,7 @@ __global__ __launch_bounds__(64 * kXmNW) void k_xm(const uint8_t *__restrict__ w
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
             const uint8_t *buf = wbuf + rt * X::kBuf;
-            wc[rt].step(buf, r16, q, b, h, xr, xl, P[rt], acc[rt], tab);
+            wc[rt].step(buf, r16, q, b, h, xr, xl, P[rt]);
             if constexpr (h == 1) wc[rt].fold(buf, r16, q, b, sm, P[rt], acc[rt]);
             if constexpr (i == 7) wc[rt].next();
             if (rt & 1) __builtin_amdgcn_sched_barrier(0);
