@@ -397,7 +397,7 @@ static hipError_t xg_go(const uint8_t *w, const _Float16 *xh, const float *us, f
 
 // Column tiles per workgroup: the fewest (rounds of one workgroup per CU) x
 // (work of one), counting one column tile's time for what a workgroup does
-// whatever its width. That picked the faster of the two in all of 159 measured
+// whatever its width. That picked the faster of the two in all of 158 measured
 // calls (3 to 16 groups, K of 512 to 4096, 256 to 1000 tokens): 8 x [1024 x
 // 4096] at 256 / 300 / 400 / 640 tokens two tiles 63 / 109 / 115 / 174 us, three
 // 69 / 73 / 132 / 148. Four do not fit the registers beside the tile sums (65
