@@ -127,13 +127,18 @@ bool workspace(DevBuf &b, size_t n, hipStream_t s) {
 // to 1 MB (Q4_K 4096 x 4096 at 16 / 60 tokens, 256 KB / 1 MB each way: 57.5 ->
 // 56.2, 126.9 -> 126.7 us): the copy to the buffer costs no more than the
 // runtime's own staging, so there is no smaller line to draw.
-// Buffers of kPinBytes, one per thread that calls; a thread that ends returns
-// its buffer to the free list, so there are never more than threads that
-// called at the same time.
+// Buffers of kPinBytes, one per thread that calls; a thread that ends gives its
+// buffer to the free list for the next one, or back to the runtime when the
+// list holds kPinKeep (16 MB) already.
 constexpr size_t kPinBytes = (size_t)1 << 20;
+constexpr size_t kPinKeep = 16;
 std::mutex g_pin_mu;
 // never destroyed (as g_scratch_map): the HIP runtime may be gone by then
-auto *g_pin_free = new std::vector<uint8_t *>();
+auto *g_pin_free = [] {
+    auto *v = new std::vector<uint8_t *>();
+    v->reserve(kPinKeep);  // so that a thread's end allocates nothing
+    return v;
+}();
 struct PinBuf {
     uint8_t *p = nullptr;
     uint8_t *get() {
@@ -155,8 +160,14 @@ struct PinBuf {
     }
     ~PinBuf() {
         if (!p) return;
-        std::lock_guard<std::mutex> lk(g_pin_mu);
-        g_pin_free->push_back(p);
+        {
+            std::lock_guard<std::mutex> lk(g_pin_mu);
+            if (g_pin_free->size() < kPinKeep) {
+                g_pin_free->push_back(p);
+                return;
+            }
+        }
+        (void)hipHostFree(p);  // (every call has waited for its copies)
     }
 };
 

@@ -15,7 +15,9 @@ its kernels on the rayon pool, parallel.rs:37-54):
   the stream still works;
 * 2 threads enqueue the same workspace-using calls on hipStreamPerThread (one
   handle value, a different stream in each thread): each thread gets a
-  workspace set of its own, and results are bit-identical to serial calls.
+  workspace set of its own, and results are bit-identical to serial calls;
+* 20 threads hold a staging buffer at once, more than are kept when they end,
+  and others after them call with what was kept.
 ctypes releases the GIL around each library call, so the calls overlap."""
 import threading
 
@@ -259,3 +261,28 @@ def test_dev_calls_on_stream_per_thread_from_two_threads(hip):
         return run
 
     _run_threads([worker(0), worker(1)])
+
+
+def test_more_threads_than_staging_buffers_are_kept(hip, oracle):
+    hip.init(0)
+    n, o = 512, 256
+    w = synth.weight(G.Q8_0, o, n, 1400)
+    hip.register_weights(w, G.Q8_0, n)
+    try:
+        for _ in range(2):
+            barrier = threading.Barrier(20)
+
+            def worker(i):
+                def run():
+                    x = synth.activations(1 + i % 3, n, 1410 + i).reshape(-1)
+                    rc, want = oracle.matmul_quant_f32(w, x, 1 + i % 3, n, o, int(G.Q8_0))
+                    assert rc == 0
+                    for k in range(2):
+                        got = np.full(want.size, np.nan, np.float32)
+                        hip.matmul_quant_f32(got, w, x, 1 + i % 3, n, o, G.Q8_0)
+                        assert rel_err(got, want) <= REL_TOL
+                        barrier.wait(timeout=60)  # every thread holds its buffer here
+                return run
+            _run_threads([worker(i) for i in range(20)])
+    finally:
+        hip.release_weights()
